@@ -633,14 +633,20 @@ namespace {
 struct Builder {
   Schedule &S;
 
+  // threads for the colour points of one interior row of B
+  static int row_threads(const DevBox &B, int pts) {
+    return ((B.n[0] - 2 * B.R + B.nc - 1) / B.nc + pts - 1) / pts;
+  }
+
   // threads per row of a level: colour points per interior row (colour
   // passes) or slots per colour row (whole-row kernels)
-  static int per_row(const Hier &H, int level, bool subrows) {
+  // (pts: colour points a thread takes)
+  static int per_row(const Hier &H, int level, bool subrows, int pts = 1) {
     const int f = H.geo.level_first[size_t(level)], n = H.geo.level_count[size_t(level)];
     int m = 0;
     for (int b = f; b < f + n; ++b) {
       const DevBox &B = H.hbox[size_t(b)];
-      m = std::max(m, subrows ? B.rl : (B.n[0] - 2 * B.R + B.nc - 1) / B.nc);
+      m = std::max(m, subrows ? B.rl : row_threads(B, pts));
     }
     return m;
   }
@@ -650,13 +656,14 @@ struct Builder {
   // (pr: the level's longest row in threads; a launch runs min(pr,
   // threads) threads per row, splitting longer rows into segments)
   static void row_blocks(const Hier &H, int level, unsigned long long *norm, bool subrows, int pr,
-                         std::vector<RowBlock> &out, int threads = kRowThreads, int reps = 1) {
+                         std::vector<RowBlock> &out, int threads = kRowThreads, int reps = 1,
+                         int pts = 1) {
     const int seg = std::min(pr, threads);
     const int rpb = std::max(1, threads / seg) * reps;
     const int f = H.geo.level_first[size_t(level)], n = H.geo.level_count[size_t(level)];
     for (int b = f; b < f + n; ++b) {
       const DevBox &B = H.hbox[size_t(b)];
-      const int len = subrows ? B.rl : (B.n[0] - 2 * B.R + B.nc - 1) / B.nc;
+      const int len = subrows ? B.rl : row_threads(B, pts);
       const int nseg = (len + seg - 1) / seg;
       const int rows = interior_rows(B) * (subrows ? B.nc : 1) * nseg;
       for (int r0 = 0; r0 < rows; r0 += rpb)
@@ -673,7 +680,7 @@ struct Builder {
     long long nb = 0;
     for (int b = f; b < f + n; ++b) {
       const DevBox &B = H.hbox[size_t(b)];
-      const int len = subrows ? B.rl : (B.n[0] - 2 * B.R + B.nc - 1) / B.nc;
+      const int len = subrows ? B.rl : row_threads(B, 1);
       const long long rows = (long long)interior_rows(B) * (subrows ? B.nc : 1) * ((len + seg - 1) / seg);
       nb += (rows + rpb - 1) / rpb;
     }
@@ -733,8 +740,9 @@ struct Builder {
         return H.slot(norm_slot >= 0 ? norm_slot : post ? Hier::slot_post(l) : Hier::slot_pre(l));
       };
       int pc = 0, ps = 0;  // threads per row: colour passes, whole-row kernels
+      const int pts = mixed ? 1 : sweep_points(eq);
       for (int h : g.second) {
-        pc = std::max(pc, per_row(*M[size_t(h)], lv[size_t(h)], false));
+        pc = std::max(pc, per_row(*M[size_t(h)], lv[size_t(h)], false, pts));
         ps = std::max(ps, per_row(*M[size_t(h)], lv[size_t(h)], true));
       }
       std::vector<RowBlock> cb, sb;
@@ -753,7 +761,7 @@ struct Builder {
       for (int h : g.second) {
         const Hier &H = *M[size_t(h)];
         const int l = lv[size_t(h)];
-        row_blocks(H, l, mixed ? nullptr : slot(H, l), false, pc, cb, threads);
+        row_blocks(H, l, mixed ? nullptr : slot(H, l), false, pc, cb, threads, 1, pts);
         if (mixed) row_blocks(H, l, slot(H, l), true, ps, sb, kRowThreads, sreps);
         for (int b = 0; b < H.geo.level_count[size_t(l)]; ++b)
           boxes.insert(H.dbox + H.geo.level_first[size_t(l)] + b);

@@ -483,6 +483,142 @@ __device__ __forceinline__ void smooth_rows(const RowBlock &Bk, ConstBox &B, uns
   wave_norm(Bk.norm, rmax);
 }
 
+// Two colour points a thread: slots t and t + 1 of a colour row (i and
+// i + NC), every field read 16 bytes a lane.  A wave's 8-byte load occupies
+// the vector memory unit for as long as its 16-byte load (16.4 cycles each,
+// measured on L1- and L2-resident data, aligned or not), and one point a
+// thread kept that unit 77% busy (N=161, 6th order: 22 loads a wave).
+// k_smooth<6,1> over the N=161 workload's launches 58.8 -> 51.4 us, <8,0>
+// at N=129 11.8 -> 10.1 us, <4,0> in a batch of 16 at N=65 21.7 -> 19.5 us.
+// The x neighbours of colour c + m of both points are three consecutive slots
+// (x + m - NC, x + m, x + m + NC).  Each point's arithmetic is smooth_rows',
+// operation for operation.
+__device__ __forceinline__ void ld_pair(const void *base, unsigned off, double &a, double &b) {
+  typedef double V2 __attribute__((ext_vector_type(2), aligned(8)));
+  const V2 v = *(const __attribute__((address_space(1))) V2 *)((const gchar *)base + off);
+  a = v.x;
+  b = v.y;
+}
+__device__ __forceinline__ void st_pair(void *base, unsigned off, double a, double b) {
+  typedef double V2 __attribute__((ext_vector_type(2), aligned(8)));
+  V2 v;
+  v.x = a;
+  v.y = b;
+  *(__attribute__((address_space(1))) V2 *)((gchar *)base + off) = v;
+}
+
+// Laplacian terms of the points at byte offsets o and o + 8 (u00, u01 their
+// u), NC = ORD / 2 + 1 colours
+template <int ORD>
+__device__ __forceinline__ void lap_pair(const void *u, unsigned o, const Nbr<ORD / 2 + 1> &n,
+                                         double u00, double u01, double ix2, double iy2, double iz2,
+                                         double l[2]) {
+  constexpr int R = ORD / 2, NC = R + 1;
+  double sx[2][4] = {}, sy[2][4] = {}, sz[2][4] = {};
+  double xv[R][3];  // [m - 1]: u at x + m - NC, x + m, x + m + NC
+#pragma unroll
+  for (int m = 1; m <= R; ++m) {
+    ld_pair(u, o + n.xm[NC - m - 1], xv[m - 1][0], xv[m - 1][1]);
+    xv[m - 1][2] = ld<double>(u, o + n.xp[m - 1] + 8u);
+    double p0, p1, m0, m1;
+    ld_pair(u, o + n.yp[m - 1], p0, p1);
+    ld_pair(u, o + n.ym[m - 1], m0, m1);
+    sy[0][m - 1] = p0 + m0;
+    sy[1][m - 1] = p1 + m1;
+    ld_pair(u, o + n.zp[m - 1], p0, p1);
+    ld_pair(u, o + n.zm[m - 1], m0, m1);
+    sz[0][m - 1] = p0 + m0;
+    sz[1][m - 1] = p1 + m1;
+  }
+#pragma unroll
+  for (int m = 1; m <= R; ++m)
+#pragma unroll
+    for (int q = 0; q < 2; ++q) sx[q][m - 1] = xv[m - 1][q + 1] + xv[NC - m - 1][q];
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const double u0 = q ? u01 : u00;
+    l[q] = star_sum<ORD, double>(star<ORD, double>(u0, sx[q][0], sx[q][1], sx[q][2], sx[q][3]),
+                                 star<ORD, double>(u0, sy[q][0], sy[q][1], sy[q][2], sy[q][3]),
+                                 star<ORD, double>(u0, sz[q][0], sz[q][1], sz[q][2], sz[q][3]), ix2,
+                                 iy2, iz2);
+  }
+}
+
+template <int ORD, int EQ>
+__device__ __forceinline__ void smooth_pairs(const RowBlock &Bk, ConstBox &B, unsigned per_row,
+                                             float inv_per_row, int colour) {
+  constexpr int R = ORD / 2, NC = R + 1;
+  const unsigned lr = fast_div(threadIdx.x, per_row, inv_per_row);
+  unsigned t = threadIdx.x - lr * per_row;
+  const int col = B.flip ? NC - 1 - colour : colour;
+  double rmax = 0.0;
+  unsigned row = unsigned(Bk.row0) + lr;
+  if (lr < unsigned(Bk.rows)) {
+    if (Bk.nseg > 1) {
+      const unsigned seg = row % unsigned(Bk.nseg);
+      row /= unsigned(Bk.nseg);
+      t += seg * per_row;
+    }
+    int j, k;
+    row_jk<R>(B, row, j, k);
+    const int first = R + int(unsigned(col + NC * 3 * kMaxAxisPoints - j - k - R) % NC);
+    const int i = first + int(2 * t) * NC;
+    if (i < B.n[0] - R) {
+      // the second point may be a ghost or padding slot: its loads stay
+      // inside the field (rows and planes follow every interior row), and
+      // it is neither written nor counted
+      const bool two = i + NC < B.n[0] - R;
+      const unsigned p = unsigned(col) * unsigned(B.cs) + unsigned(k) * unsigned(B.ps) +
+                         unsigned(j) * unsigned(B.rs) + unsigned(first / NC) + 2 * t;
+      const Nbr<NC> nb = box_offs<NC, 8>(B, col, first % NC);
+      const unsigned o = p * 8u;
+      double *u = B.f[F_U];
+      double rho[2] = {0.0, 0.0};
+      // rho is +0 outside the rho box: a pair that reaches into it is read
+      // whole
+      if ((unsigned(j - B.rlo[1]) < unsigned(B.rhi[1] - B.rlo[1])) &
+          (unsigned(k - B.rlo[2]) < unsigned(B.rhi[2] - B.rlo[2])) & (i + NC >= B.rlo[0]) &
+          (i < B.rhi[0]))
+        ld_pair(B.f[F_RHO], o, rho[0], rho[1]);
+      double u0[2], lu[2], b[2], c[2], d[2] = {0.0, 0.0}, e[2] = {0.0, 0.0};
+      ld_pair(u, o, u0[0], u0[1]);
+      ld_pair(B.f[F_B], o, b[0], b[1]);
+      ld_pair(B.f[F_C], o, c[0], c[1]);
+      if constexpr (EQ == 1) {
+        ld_pair(B.f[F_D], o, d[0], d[1]);
+        ld_pair(B.f[F_E], o, e[0], e[1]);
+      }
+      lap_pair<ORD>(u, o, nb, u0[0], u0[1], B.idx2[0], B.idx2[1], B.idx2[2], lu);
+      double un[2];
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        double N, dN;
+        nonlinear<EQ>(lu[q], B.dulap, b[q], c[q] + u0[q], d[q], e[q], N, dN);
+        const double res = N - rho[q];
+        un[q] = u0[q] - res / dN;
+        if (q == 0 || two) {
+          rmax = fmax(rmax, fabs(res));
+          if (!(un[q] == un[q])) rmax = __longlong_as_double(0x7ff0000000000000LL);
+        }
+      }
+      if (two)
+        st_pair(u, o, un[0], un[1]);
+      else
+        st<double>(u, o, un[0]);
+    }
+  }
+  wave_norm(Bk.norm, rmax);
+}
+
+template <int ORD, int EQ>
+__device__ __forceinline__ void smooth_block(const RowBlock &Bk, ConstBox &B, unsigned per_row,
+                                             float inv_per_row, int colour) {
+  if constexpr (sweep_points(EQ) == 2)
+    smooth_pairs<ORD, EQ>(Bk, B, per_row, inv_per_row, colour);
+  else
+    smooth_rows<ORD, EQ>(Bk, B, per_row, inv_per_row, colour);
+}
+
 // box1: the one box of every listed block, when the launch covers a single
 // box (else null); its descriptor is then fetched without waiting for the
 // block's.  Either way the descriptor's cache lines are fetched in one batch
@@ -495,11 +631,11 @@ __global__ __launch_bounds__(kMaxRowThreads) void k_smooth(const RowBlock *__res
   if (box1) {
     const RowBlock Bk = blocks[xcd_block()];
     fetch_box(box1);
-    smooth_rows<ORD, EQ>(Bk, cbox(box1), per_row, inv_per_row, colour);
+    smooth_block<ORD, EQ>(Bk, cbox(box1), per_row, inv_per_row, colour);
   } else {
     const RowBlock Bk = blocks[xcd_block()];
     fetch_box(Bk.box);
-    smooth_rows<ORD, EQ>(Bk, cbox(Bk.box), per_row, inv_per_row, colour);
+    smooth_block<ORD, EQ>(Bk, cbox(Bk.box), per_row, inv_per_row, colour);
   }
 }
 

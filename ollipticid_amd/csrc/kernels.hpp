@@ -195,6 +195,10 @@ struct RowBlock {
   int nseg;
 };
 constexpr int kRowThreads = 256;  // threads per row workgroup
+// colour points of a row a thread of the FP64 colour passes takes: two
+// adjacent ones, except for Punctures_EM, whose first derivatives read
+// their neighbours one by one
+constexpr int sweep_points(int eq) { return eq == kEqPuncturesEm ? 1 : 2; }
 // the colour passes (k_smooth, k_smooth32) take 64..kMaxRowThreads threads
 // per workgroup, a multiple of 64 picked per (precision, order) by the
 // launch-shape table (sweep_threads); their results do not depend on it
