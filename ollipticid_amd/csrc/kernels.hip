@@ -345,18 +345,35 @@ __device__ __forceinline__ double wave_max_dpp(double v) {
   return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
 }
 
+// what the block's norm slot holds as the block starts (thread 0; 0 without
+// a slot).  The slot only grows, so wave_norm leaves the atomic out when the
+// block's maximum is no larger: after a phase's first sweep that is nearly
+// every block.  An atomic per block on 16 lines cost a colour pass of one
+// N=65 box 0.5 us of 4.4.  Only launches of small workgroups (sweep_rule)
+// read it: in longer launches the atomics overlap the passes, and the load
+// would cost 2%.
+__device__ __forceinline__ double norm_seen(const unsigned long long *slot) {
+  if (blockDim.x > kFewRowThreads || threadIdx.x != 0 || !slot) return 0.0;
+  return ld<double>(slot, (blockIdx.x & (kNormSubSlots - 1)) * (kNormStride * 8u));
+}
+
 // block max of v (every thread must call; blockDim.x a multiple of 64, at
-// most kMaxRowThreads), one norm update per block
-__device__ __forceinline__ void wave_norm(unsigned long long *slot, double v) {
+// most kMaxRowThreads), at most one norm update per block: none when the
+// slot already held `seen` >= the maximum
+__device__ __forceinline__ void wave_norm(unsigned long long *slot, double v, double seen) {
   __shared__ double sh[kMaxRowThreads / 64];
   const double m = wave_max_dpp(v);
+  if (blockDim.x == 64) {
+    if (threadIdx.x == 0 && slot && m > seen) norm_update(slot, m);
+    return;
+  }
   if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = m;
   __syncthreads();
   if (threadIdx.x == 0 && slot) {
     double b = sh[0];
     const int nw = int(blockDim.x >> 6);
     for (int w = 1; w < nw; ++w) b = fmax(b, sh[w]);
-    if (b > 0.0) norm_update(slot, b);
+    if (b > seen) norm_update(slot, b);
   }
 }
 
@@ -462,6 +479,7 @@ __device__ __forceinline__ void smooth_rows(const RowBlock &Bk, ConstBox &B, uns
   constexpr int NC = colours_of(ORD, EQ);
   const unsigned lr = fast_div(threadIdx.x, per_row, inv_per_row);
   const int t = int(threadIdx.x - lr * per_row);
+  const double seen = norm_seen(Bk.norm);
   double rmax = 0.0;
   unsigned p;
   int s, i, j, k;
@@ -480,7 +498,7 @@ __device__ __forceinline__ void smooth_rows(const RowBlock &Bk, ConstBox &B, uns
     rmax = fabs(res);
     if (!(un == un)) rmax = __longlong_as_double(0x7ff0000000000000LL);  // inf flags NaN
   }
-  wave_norm(Bk.norm, rmax);
+  wave_norm(Bk.norm, rmax, seen);
 }
 
 // Two colour points a thread: slots t and t + 1 of a colour row (i and
@@ -551,6 +569,7 @@ __device__ __forceinline__ void smooth_pairs(const RowBlock &Bk, ConstBox &B, un
   const unsigned lr = fast_div(threadIdx.x, per_row, inv_per_row);
   unsigned t = threadIdx.x - lr * per_row;
   const int col = B.flip ? NC - 1 - colour : colour;
+  const double seen = norm_seen(Bk.norm);
   double rmax = 0.0;
   unsigned row = unsigned(Bk.row0) + lr;
   if (lr < unsigned(Bk.rows)) {
@@ -607,7 +626,7 @@ __device__ __forceinline__ void smooth_pairs(const RowBlock &Bk, ConstBox &B, un
         st<double>(u, o, un[0]);
     }
   }
-  wave_norm(Bk.norm, rmax);
+  wave_norm(Bk.norm, rmax, seen);
 }
 
 template <int ORD, int EQ>
@@ -734,6 +753,7 @@ __global__ __launch_bounds__(kFusedThreads) void k_smooth_fused(const TileBlock 
   const void *X = parity ? B.f[F_R] : B.f[F_U];
   void *Y = parity ? B.f[F_U] : B.f[F_R];
   const int nt = T.ty * T.tz;
+  const double seen = norm_seen(T.norm);
   double rmax;
   if constexpr (PAIR) {
     int yb, ya, zb, za;
@@ -747,7 +767,7 @@ __global__ __launch_bounds__(kFusedThreads) void k_smooth_fused(const TileBlock 
   } else {
     rmax = fused_pass<ORD, EQ, Q>(T, B, X, Y, nt, 0, 0, 0);
   }
-  wave_norm(T.norm, rmax);
+  wave_norm(T.norm, rmax, seen);
 }
 
 // operator on the interior: mode RES_OPERATOR r = N(u), RES_DEFECT
@@ -760,6 +780,7 @@ __global__ __launch_bounds__(kRowThreads) void k_residual(const RowBlock *__rest
   constexpr int NC = colours_of(ORD, EQ);
   const RowBlock Bk = blocks[xcd_block()];
   ConstBox &B = cbox(Bk.box);
+  const double seen = norm_seen(Bk.norm);
   double rmax = 0.0;
   for_rows(Bk, per_row, inv_per_row, [&](unsigned rpb, unsigned lr0) {
     unsigned p;
@@ -777,7 +798,7 @@ __global__ __launch_bounds__(kRowThreads) void k_residual(const RowBlock *__rest
       st<double>(B.f[F_R], o, mode == RES_DERIVATIVE ? dN : N);
     rmax = nan_max(rmax, fabs(N));
   });
-  wave_norm(Bk.norm, rmax);
+  wave_norm(Bk.norm, rmax, seen);
 }
 
 // ------------------------------------------------------------------
@@ -796,6 +817,7 @@ __global__ __launch_bounds__(kRowThreads) void k_defect32(const RowBlock *__rest
   constexpr int NC = colours_of(ORD, EQ);
   const RowBlock Bk = blocks[xcd_block()];
   ConstBox &B = cbox(Bk.box);
+  const double seen = norm_seen(Bk.norm);
   double rmax = 0.0;
   for_rows(Bk, per_row, inv_per_row, [&](unsigned rpb, unsigned lr0) {
     unsigned p;
@@ -814,7 +836,7 @@ __global__ __launch_bounds__(kRowThreads) void k_defect32(const RowBlock *__rest
     rmax = nan_max(rmax, fabs(res));
     if (!(res == res)) rmax = __longlong_as_double(0x7ff0000000000000LL);
   });
-  wave_norm(Bk.norm, rmax);
+  wave_norm(Bk.norm, rmax, seen);
 }
 
 template <int ORD>
