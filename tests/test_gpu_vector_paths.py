@@ -33,3 +33,18 @@ def test_paired_sweeps(eq, n, order):
         for ib in s.level_boxes(lv):
             assert rel_err(h.get_field(ib, oa.F_U), s.field(ib, O.F_U)) < 1e-12, (lv, ib)
     h.close()
+
+
+@pytest.mark.parametrize("eq", [0, 1])
+@pytest.mark.parametrize("n", [25, 33, 41])  # coarsest boxes 13^3, 17^3, 21^3
+def test_coarsest_solve(eq, n):
+    """One FAS step: the coarsest box with its faces, edges and corners, and
+    every finer box that reads them."""
+    h, s = pair(argv(eq, n, 2))
+    top = s.levels - 1
+    for _ in range(2):
+        ng, no = h.fas(top), s.fasn(top)
+        assert abs(ng - no) <= 1e-9 * no, (ng, no)
+        for ib in range(s.nbox):
+            assert rel_err(h.get_field(ib, oa.F_U), s.field(ib, O.F_U)) < 1e-12, ib
+    h.close()
