@@ -33,8 +33,8 @@ def build(verbose=True):
     geo_o = os.path.join(objdir, "geometry.o")
     _run(["g++"] + HOST_FLAGS + ["-c", os.path.join(CSRC, "geometry.cpp"), "-o", geo_o])
     objs = [geo_o]
-    for src in ("kernels.hip", "engine.hip", "capi.hip"):
-        o = os.path.join(objdir, src.replace(".hip", ".o"))
+    for src in ("kernels.hip", "engine.hip", "capi.hip", "staging.cpp"):
+        o = os.path.join(objdir, os.path.splitext(src)[0] + ".o")
         _run([HIPCC] + DEVICE_FLAGS + ["-c", os.path.join(CSRC, src), "-o", o])
         objs.append(o)
     tmp = LIB + ".tmp"

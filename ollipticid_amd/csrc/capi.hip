@@ -16,6 +16,7 @@
 
 #include "../../include/olliptic_amd.h"
 #include "engine.hpp"
+#include "staging.hpp"
 
 using namespace oll;
 
@@ -84,6 +85,8 @@ struct oll_hier {
   Timing timing;
   double last_ms = 0;
   bool graphs = true;
+  oll_hier() { staging_retain(); }
+  ~oll_hier() { staging_release(); }
 };
 
 namespace {
@@ -242,16 +245,7 @@ int oll_get_field(oll_hier *h, int ibox, int field, double *host) {
   if (!h || !host) return fail(OLL_EINVAL, "null argument");
   if (ibox < 0 || ibox >= int(h->H.hbox.size()) || field < 0 || field >= fields_of(h->H.prob.eq))
     return fail(OLL_EINVAL, "box or field out of range");
-  const DevBox &b = h->H.hbox[size_t(ibox)];
-  std::vector<double> st(size_t(b.size));
-  CAPI_CHECK(hipMemcpyAsync(st.data(), b.f[field], st.size() * sizeof(double),
-                            hipMemcpyDeviceToHost, h->stream));
-  CAPI_CHECK(hipStreamSynchronize(h->stream));
-  // colour blocks -> plain lexicographic order (i fastest)
-  size_t q = 0;
-  for (int k = 0; k < b.n[2]; ++k)
-    for (int j = 0; j < b.n[1]; ++j)
-      for (int i = 0; i < b.n[0]; ++i) host[q++] = st[size_t(pidx(b, i, j, k))];
+  CAPI_RC(field_host(h->H, h->stream, ibox, field, host, true, e_));
   return OLL_OK;
 }
 
@@ -259,15 +253,7 @@ int oll_set_field(oll_hier *h, int ibox, int field, const double *host) {
   if (!h || !host) return fail(OLL_EINVAL, "null argument");
   if (ibox < 0 || ibox >= int(h->H.hbox.size()) || field < 0 || field >= fields_of(h->H.prob.eq))
     return fail(OLL_EINVAL, "box or field out of range");
-  const DevBox &b = h->H.hbox[size_t(ibox)];
-  std::vector<double> st(size_t(b.size), 0.0);
-  size_t q = 0;
-  for (int k = 0; k < b.n[2]; ++k)
-    for (int j = 0; j < b.n[1]; ++j)
-      for (int i = 0; i < b.n[0]; ++i) st[size_t(pidx(b, i, j, k))] = host[q++];
-  CAPI_CHECK(hipMemcpyAsync(b.f[field], st.data(), st.size() * sizeof(double),
-                            hipMemcpyHostToDevice, h->stream));
-  CAPI_CHECK(hipStreamSynchronize(h->stream));
+  CAPI_RC(field_host(h->H, h->stream, ibox, field, const_cast<double *>(host), false, e_));
   if (field == F_RHO) {  // the caller's rho may be nonzero anywhere in the box
     std::string err;
     const int rc = hier_rho_whole(h->H, ibox, 1, h->stream, err);
@@ -542,6 +528,8 @@ struct oll_engine {
   // the host), admissions; rebuild count
   double build_ms = 0, run_ms = 0, admit_ms = 0;
   long long rebuilds = 0;
+  oll_engine() { staging_retain(); }
+  ~oll_engine() { staging_release(); }
 };
 
 namespace {

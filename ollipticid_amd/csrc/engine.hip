@@ -9,6 +9,8 @@
 #include <set>
 #include <tuple>
 
+#include "staging.hpp"
+
 // host arithmetic that must equal the reference's (coordinates, the
 // approximation's puncture values) is rounded operation by operation
 #pragma clang fp contract(off)
@@ -478,6 +480,8 @@ void hier_release(Hier &H) {
   (void)hipFree(H.dxfer);
   (void)hipFree(H.norms);
   (void)hipFree(H.iters);
+  (void)hipFree(H.interp_scratch);
+  H.interp_scratch = nullptr;
   H.slab = nullptr;
   H.slab32 = nullptr;
   H.dbox = nullptr;
@@ -1512,21 +1516,111 @@ void puncture_approx(const Hier &H, double *u_at_p) {
   }
 }
 
+// a borrowed Staging, returned on every path once the stream is done with it
+struct StagingUse {
+  hipStream_t s;
+  Staging *g = staging_take();
+  hipEvent_t ev[2] = {nullptr, nullptr};
+  explicit StagingUse(hipStream_t stream) : s(stream) {}
+  ~StagingUse() {
+    (void)hipStreamSynchronize(s);
+    for (hipEvent_t e : ev)
+      if (e) (void)hipEventDestroy(e);
+    staging_give(g);
+  }
+  hipError_t events() {
+    for (hipEvent_t &e : ev) {
+      const hipError_t rc = hipEventCreateWithFlags(&e, hipEventDisableTiming);
+      if (rc != hipSuccess) return rc;
+    }
+    return hipSuccess;
+  }
+};
+
+// One half of the staging is filled or drained by the GPU while the host
+// copies the other: fields of one half's size take one launch and one copy
+int field_host(Hier &H, hipStream_t s, int ibox, int field, double *host, bool to_host,
+               std::string &err) {
+  const DevBox &b = H.hbox[size_t(ibox)];
+  const size_t np = size_t(npts(b)), half = Staging::kBytes / sizeof(double);
+  const size_t chunks = (np + half - 1) / half;
+  StagingUse use(s);
+  if (!use.g) return err = "pinned staging memory", OLL_ENOMEM;
+  if (chunks > 1) ENG_CHECK(use.events());
+  auto begin = [&](size_t c) { return c * half; };
+  auto count = [&](size_t c) { return std::min(half, np - c * half); };
+  auto buf = [&](size_t c) { return reinterpret_cast<double *>(use.g->half[c & 1]); };
+  // to the host: chunk c is copied out while chunk c + 1 is written; from
+  // it: chunk c is copied in while chunk c - 1 is read
+  for (size_t c = 0; c < chunks + (to_host ? 1 : 0); ++c) {
+    if (!to_host) {
+      if (c >= 2) ENG_CHECK(hipEventSynchronize(use.ev[c & 1]));
+      host_copy(buf(c), host + begin(c), count(c) * sizeof(double));
+    }
+    if (c < chunks) {
+      launch_field_host(s, b, field, buf(c), unsigned(begin(c)), unsigned(count(c)), to_host);
+      ENG_CHECK(hipGetLastError());
+      if (chunks > 1) ENG_CHECK(hipEventRecord(use.ev[c & 1], s));
+    }
+    if (to_host && c > 0) {
+      if (chunks > 1)
+        ENG_CHECK(hipEventSynchronize(use.ev[(c - 1) & 1]));
+      else
+        ENG_CHECK(hipStreamSynchronize(s));
+      host_copy(host + begin(c - 1), buf(c - 1), count(c - 1) * sizeof(double));
+    }
+  }
+  ENG_CHECK(hipStreamSynchronize(s));
+  return OLL_OK;
+}
+
 int interp_points(Hier &H, hipStream_t s, int field, int npts, const int *box, const double *xyz,
                   int ord, double *out, std::string &err) {
   if (npts <= 0) return OLL_OK;
-  int *d_box = nullptr;
-  double *d_xyz = nullptr, *d_out = nullptr;
-  TempBuffers tmp;
-  ENG_CHECK(tmp.alloc(&d_box, size_t(npts)));
-  ENG_CHECK(tmp.alloc(&d_xyz, size_t(3 * npts)));
-  ENG_CHECK(tmp.alloc(&d_out, size_t(npts)));
-  ENG_CHECK(hipMemcpyAsync(d_box, box, size_t(npts) * sizeof(int), hipMemcpyHostToDevice, s));
-  ENG_CHECK(hipMemcpyAsync(d_xyz, xyz, size_t(3 * npts) * sizeof(double), hipMemcpyHostToDevice, s));
-  launch_interp_points(s, H.dbox, field, d_box, d_xyz, npts, ord, d_out);
-  ENG_CHECK(hipGetLastError());
-  ENG_CHECK(hipMemcpyAsync(out, d_out, size_t(npts) * sizeof(double), hipMemcpyDeviceToHost, s));
-  ENG_CHECK(hipStreamSynchronize(s));
+  // a half of the staging holds a chunk's coordinates, boxes and values; the
+  // host copies one half while the GPU works on the other (two chunks or
+  // more where there are many points).  The kernel writes the values to the
+  // pinned half and reads few points from it; many are first copied to the
+  // handle's device scratch, which the chunks share on the stream (reading
+  // 28 bytes a point over PCIe would take longer than interpolating).
+  constexpr size_t kIn = 3 * sizeof(double) + sizeof(int), kPoint = kIn + sizeof(double);
+  constexpr size_t kMost = Staging::kBytes / kPoint / 64 * 64;
+  constexpr size_t kFew = 4096, kSplit = 65536;
+  const size_t n = size_t(npts);
+  const size_t half = n <= kSplit ? n : std::min(kMost, (n + 127) / 128 * 64);
+  const size_t chunks = (n + half - 1) / half;
+  const bool direct = n <= kFew;
+  if (!direct && !H.interp_scratch) {
+    ENG_CHECK(hipMalloc(reinterpret_cast<void **>(&H.interp_scratch), kMost * kIn));
+    H.bytes += kMost * kIn;
+  }
+  StagingUse use(s);
+  if (!use.g) return err = "pinned staging memory", OLL_ENOMEM;
+  if (chunks > 1) ENG_CHECK(use.events());
+  for (size_t c = 0; c <= chunks; ++c) {
+    if (c < chunks) {
+      const size_t b0 = c * half, m = std::min(half, n - b0);
+      char *hb = use.g->half[c & 1];
+      double *vals = reinterpret_cast<double *>(hb);  // values, coordinates, boxes
+      char *in = hb + m * sizeof(double);
+      host_copy(in, xyz + 3 * b0, 3 * m * sizeof(double));
+      host_copy(in + 3 * m * sizeof(double), box + b0, m * sizeof(int));
+      char *src = direct ? in : H.interp_scratch;
+      if (!direct) ENG_CHECK(hipMemcpyAsync(src, in, m * kIn, hipMemcpyHostToDevice, s));
+      launch_interp_points(s, H.dbox, field, reinterpret_cast<const int *>(src + 3 * m * sizeof(double)),
+                           reinterpret_cast<const double *>(src), int(m), ord, vals);
+      ENG_CHECK(hipGetLastError());
+      if (chunks > 1) ENG_CHECK(hipEventRecord(use.ev[c & 1], s));
+    }
+    if (c > 0) {
+      const size_t b0 = (c - 1) * half, m = std::min(half, n - b0);
+      if (chunks > 1)
+        ENG_CHECK(hipEventSynchronize(use.ev[(c - 1) & 1]));
+      else
+        ENG_CHECK(hipStreamSynchronize(s));
+      host_copy(out + b0, use.g->half[(c - 1) & 1], m * sizeof(double));
+    }
+  }
   return OLL_OK;
 }
 

@@ -52,6 +52,7 @@ struct Hier {
   unsigned long long *norms = nullptr;  // nslots * kNormWords
   int nslots = 0;
   int *iters = nullptr;
+  char *interp_scratch = nullptr;  // interp_points' device chunk, on first use
   PunctureArgs pa{};
   double eps_solv = 0, eps_coarse = 0, coarse_omega = 1;
   std::vector<std::vector<double>> colour_pts;  // [level][colour]
@@ -201,6 +202,10 @@ int adm_mass_with(Hier &H, hipStream_t s, const AdmBuffers &d, double *puncture,
                   std::string &err);
 // elliptic.cc:2232-2444 Get_Puncture_App values (host arithmetic)
 void puncture_approx(const Hier &H, double *u_at_p);
+// one field of box ibox to (or from) a host array in lexicographic order (i
+// fastest); waits for it
+int field_host(Hier &H, hipStream_t s, int ibox, int field, double *host, bool to_host,
+               std::string &err);
 // Lagrange interpolation of `field` at npts host points (box[q], xyz[3q..3q+2])
 int interp_points(Hier &H, hipStream_t s, int field, int npts, const int *box, const double *xyz,
                   int ord, double *out, std::string &err);

@@ -3008,55 +3008,159 @@ __global__ __launch_bounds__(256) void k_adm_sphere(const DevBox *__restrict__ b
   sph[(long long)box * nt * nt + q] = v * sin(th);
 }
 
+// Points q0 .. q0 + n - 1 of one field of a box, lexicographic (i fastest),
+// to or from `host` (pinned memory the GPU reaches over PCIe), the colour
+// blocks' order undone or made on the way.  Bound by PCIe: a wave's 512
+// bytes of `host` are contiguous, its NC runs in the colour blocks 128 bytes
+// each.  A host loop over the colour blocks' index map took 14.8 ms for the
+// 4.5 M points of one N=161 box, copies included; this way 1.7 ms.
+template <bool TO_HOST>
+__global__ __launch_bounds__(256) void k_field_host(DevBox B, double *__restrict__ f,
+                                                     double *__restrict__ host, unsigned q0,
+                                                     unsigned n) {
+  const unsigned q = blockIdx.x * 256u + threadIdx.x;
+  if (q >= n) return;
+  int i, j, k;
+  point_ijk(B, (long long)q0 + q, i, j, k);
+  const long long p = pidx(B, i, j, k);
+  if constexpr (TO_HOST)
+    host[q] = f[p];
+  else
+    f[p] = host[q];
+}
+
+// lane N of the caller's row of 16 lanes
+template <int N>
+__device__ __forceinline__ double row_lane(double v) {
+  return dpp_f64<0x150 + N, 0xF>(v);
+}
+template <int N>
+__device__ __forceinline__ int row_lane(int v) {
+  return __builtin_amdgcn_update_dpp(v, v, 0x150 + N, 0xF, 0xF, false);
+}
+
 // Lagrange interpolation of one field at arbitrary points (one box per
-// point), interpolation.cc:189-303
-__global__ __launch_bounds__(64) void k_interp_points(const DevBox *__restrict__ boxes, int field,
-                                                       const int *__restrict__ pbox,
-                                                       const double *__restrict__ pxyz, int npts,
-                                                       int ord, double *__restrict__ out) {
-  const int q = blockIdx.x * blockDim.x + threadIdx.x;
+// point), interpolation.cc:189-303.  16 lanes (one DPP row) a point: the
+// lanes search the axes' cells and evaluate the weights side by side, then
+// each sums the z nodes of its (x, y) column of nodes (NI = 8: x node
+// lane % 8 of two y nodes at a time; 16: up to ten x nodes, one y node), and
+// the columns are added over y and x in the reference's order through row
+// broadcasts.  One point a thread did 168 dependent divisions and 512
+// scattered loads in turn: 200,000 points at order 7 took 595 us, now 258.
+template <int NI>
+__global__ __launch_bounds__(256) void k_interp_points(const DevBox *__restrict__ boxes, int field,
+                                                        const int *__restrict__ pbox,
+                                                        const double *__restrict__ pxyz, int npts,
+                                                        int ord, double *__restrict__ out) {
+  constexpr int NMAX = NI == 8 ? 8 : 10;  // nodes per axis, at most
+  constexpr int NJ = 16 / NI;             // y nodes at a time
+  const int lane = int(threadIdx.x & 15u);
+  const int q = int(blockIdx.x * (blockDim.x / 16u) + (threadIdx.x >> 4));
   if (q >= npts) return;
   const DevBox &B = boxes[pbox[q]];
   const double *__restrict__ f = B.f[field];
   const double X[3] = {pxyz[3 * q], pxyz[3 * q + 1], pxyz[3 * q + 2]};
-  int c[3], s[3];
-  bool coinc = true;
-  for (int a = 0; a < 3; ++a) {
-    c[a] = cell_of(B, a, X[a]);
-    if (!(fabs(X[a] - coord(B, a, c[a])) <= 3 * kEps)) coinc = false;
-  }
-  if (coinc) {
-    out[q] = f[pidx(B, c[0], c[1], c[2])];
+  // lanes 0, 1, 2 of the row search axes x, y, z
+  const int ax = lane < 3 ? lane : 0;
+  const double xa = ax == 0 ? X[0] : (ax == 1 ? X[1] : X[2]);
+  const int ca = cell_of(B, ax, xa);
+  const int hit = fabs(xa - coord(B, ax, ca)) <= 3 * kEps;
+  const int c[3] = {row_lane<0>(ca), row_lane<1>(ca), row_lane<2>(ca)};
+  if (row_lane<0>(hit) & row_lane<1>(hit) & row_lane<2>(hit)) {
+    if (lane == 0) out[q] = f[pidx(B, c[0], c[1], c[2])];
     return;
   }
   // a box with fewer than ord + 1 points per axis takes the widest stencil
   // it holds (interpolation.cc:221-250 would read outside the box there)
   ord = min(ord, min(B.n[0], min(B.n[1], B.n[2])) - 1);
-  double w[3][10];
+  int s[3];
+#pragma unroll
   for (int a = 0; a < 3; ++a) {
     int s0 = (ord % 2 == 0) ? c[a] - ord / 2 : c[a] - (ord + 1) / 2;
     if (s0 < 0) s0 = 0;
     else if (s0 + ord >= B.n[a]) s0 = B.n[a] - ord - 1;
     s[a] = s0;
-    for (int m = 0; m <= ord; ++m) {
-      const double xn = coord(B, a, s0 + m);
-      double lp = 1.0;
-      for (int l = s0; l < s0 + m; ++l) lp *= (X[a] - coord(B, a, l)) / (xn - coord(B, a, l));
-      for (int l = s0 + m + 1; l <= s0 + ord; ++l) lp *= (X[a] - coord(B, a, l)) / (xn - coord(B, a, l));
-      w[a][m] = lp;
-    }
   }
+  // weight of node m of axis a at lane m of wt[a]
+  auto weight = [&](double x, double lo, double d, int s0, int m) {
+    const double xn = lo + (double)(s0 + m) * d;
+    double lp = 1.0;
+    for (int l = 0; l <= ord; ++l) {
+      const double xl = lo + (double)(s0 + l) * d;
+      const double t = (x - xl) / (xn - xl);
+      if (l != m) lp *= t;
+    }
+    return lp;
+  };
+  const int m8 = lane & 7, hi = lane >> 3;
+  double wt[3];
+  if constexpr (NI == 8) {
+    // the lower lanes weight x and then z, the upper ones y
+    const double w01 = weight(hi ? X[1] : X[0], hi ? B.lo[1] : B.lo[0], hi ? B.d[1] : B.d[0],
+                              hi ? s[1] : s[0], m8);
+    wt[0] = w01;
+    wt[1] = dpp_f64<0x128, 0xF>(w01);  // row_ror:8
+    wt[2] = weight(X[2], B.lo[2], B.d[2], s[2], m8);
+  } else {
+#pragma unroll
+    for (int a = 0; a < 3; ++a) wt[a] = weight(X[a], B.lo[a], B.d[a], s[a], lane);
+  }
+  double wz[NMAX], wy[NMAX];
+#define OLL_ROW8(F) F(0) F(1) F(2) F(3) F(4) F(5) F(6) F(7)
+#define OLL_W(m) \
+  wz[m] = row_lane<m>(wt[2]); \
+  wy[m] = row_lane<m>(wt[1]);
+  OLL_ROW8(OLL_W)
+  if constexpr (NMAX > 8) {
+    OLL_W(8)
+    OLL_W(9)
+  }
+#undef OLL_W
+  // the lane's x node (clamped: lanes past the stencil load its last node
+  // and their sums are not used)
+  const int I = min(NI == 8 ? m8 : lane, ord), Jb = NI == 8 ? hi : 0;
+  const int nc = B.nc;
+  const int xi = s[0] + I, xslot = split_div(B, xi);
+  double uj = 0.0;  // the lane's column sums over y (NI = 8: of the row's lower lanes)
+  const double *__restrict__ col0 = f + (long long)s[2] * B.ps + xslot;
+  // y nodes J0 (and J0 + 1)
+  auto columns = [&](int J0, double w0, double w1) {
+    const int yj = s[1] + min(J0 + Jb, ord);
+    int col = xi + yj + s[2];
+    col -= split_div(B, col) * nc;
+    const double *__restrict__ row = col0 + (long long)yj * B.rs;
+    double v[NMAX];
+#pragma unroll
+    for (int K = 0; K < NMAX; ++K) {
+      v[K] = 0.0;
+      if (K <= ord) v[K] = row[(long long)col * B.cs];
+      row += B.ps;
+      col = col + 1 == nc ? 0 : col + 1;
+    }
+    double uk = 0.0;
+#pragma unroll
+    for (int K = 0; K < NMAX; ++K)
+      if (K <= ord) uk += v[K] * wz[K];
+    uj += uk * w0;
+    if constexpr (NJ == 2) {
+      const double up = dpp_f64<0x128, 0xF>(uk);  // the row's other half
+      if (J0 + 1 <= ord) uj += up * w1;
+    }
+  };
+#pragma unroll
+  for (int J0 = 0; J0 < NMAX; J0 += NJ)
+    if (J0 <= ord) columns(J0, wy[J0], NJ == 2 ? wy[J0 + NJ - 1] : 0.0);
   double acc = 0.0;
-  for (int I = 0; I <= ord; ++I) {
-    double uj = 0.0;
-    for (int J = 0; J <= ord; ++J) {
-      double uk = 0.0;
-      for (int K = 0; K <= ord; ++K) uk += f[pidx(B, s[0] + I, s[1] + J, s[2] + K)] * w[2][K];
-      uj += uk * w[1][J];
-    }
-    acc += uj * w[0][I];
+#define OLL_A(m) \
+  if (m <= ord) acc += row_lane<m>(uj) * row_lane<m>(wt[0]);
+  OLL_ROW8(OLL_A)
+  if constexpr (NMAX > 8) {
+    OLL_A(8)
+    OLL_A(9)
   }
-  out[q] = acc;
+#undef OLL_A
+#undef OLL_ROW8
+  if (lane == 0) out[q] = acc;
 }
 
 __global__ void k_zero_u64(unsigned long long *p, long long n) {
@@ -3392,10 +3496,22 @@ void launch_adm_sphere(hipStream_t s, const DevBox *boxes, int nbox, const doubl
                      centres, sph, nt);
 }
 
+void launch_field_host(hipStream_t s, const DevBox &B, int field, double *host, unsigned q0,
+                       unsigned n, bool to_host) {
+  if (n == 0) return;
+  if (to_host)
+    hipLaunchKernelGGL(k_field_host<true>, dim3(ceil_div(n, 256)), dim3(256), 0, s, B, B.f[field], host, q0, n);
+  else
+    hipLaunchKernelGGL(k_field_host<false>, dim3(ceil_div(n, 256)), dim3(256), 0, s, B, B.f[field], host, q0, n);
+}
+
 void launch_interp_points(hipStream_t s, const DevBox *boxes, int field, const int *pbox,
                           const double *pxyz, int npts, int ord, double *out) {
-  hipLaunchKernelGGL(k_interp_points, dim3(ceil_div(npts, 64)), dim3(64), 0, s, boxes, field, pbox,
-                     pxyz, npts, ord, out);
+  const dim3 grid(ceil_div(npts, 16));
+  if (ord <= 7)
+    hipLaunchKernelGGL(k_interp_points<8>, grid, dim3(256), 0, s, boxes, field, pbox, pxyz, npts, ord, out);
+  else
+    hipLaunchKernelGGL(k_interp_points<16>, grid, dim3(256), 0, s, boxes, field, pbox, pxyz, npts, ord, out);
 }
 
 }  // namespace oll

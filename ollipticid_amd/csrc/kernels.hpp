@@ -499,6 +499,10 @@ void launch_adm_sphere(hipStream_t s, const DevBox *boxes, int nbox, const doubl
 // u on every point of box B set to the analytic approximation
 // (elliptic.cc:1977-2222)
 void launch_approx_box(hipStream_t s, const DevBox &B, const PunctureArgs &pa);
+// n points from lexicographic point q0 of a field of box B, to host (or from
+// it): host is pinned memory mapped into the GPU's address space
+void launch_field_host(hipStream_t s, const DevBox &B, int field, double *host, unsigned q0,
+                       unsigned n, bool to_host);
 void launch_interp_points(hipStream_t s, const DevBox *boxes, int field, const int *pbox,
                           const double *pxyz, int npts, int ord, double *out);
 

@@ -1,0 +1,95 @@
+// See staging.hpp.
+#include "staging.hpp"
+
+#include <cstring>
+#include <mutex>
+#include <new>
+#include <system_error>
+#include <thread>
+
+namespace oll {
+
+namespace {
+constexpr int kKeep = 4;
+constexpr int kCopyThreads = 4;
+constexpr size_t kThreadBytes = size_t(256) << 10;  // least share of a thread
+
+std::mutex g_mu;
+Staging *g_idle[kKeep];
+int g_nidle = 0;
+int g_handles = 0;
+
+void destroy(Staging *s) {
+  if (!s) return;
+  for (char *p : s->half)
+    if (p) (void)hipHostFree(p);
+  delete s;
+}
+}  // namespace
+
+Staging *staging_take() {
+  {
+    std::lock_guard<std::mutex> lock(g_mu);
+    if (g_nidle > 0) return g_idle[--g_nidle];
+  }
+  Staging *s = new (std::nothrow) Staging();
+  if (!s) return nullptr;
+  for (char *&p : s->half)
+    if (hipHostMalloc(reinterpret_cast<void **>(&p), Staging::kBytes, hipHostMallocPortable) != hipSuccess) {
+      p = nullptr;
+      destroy(s);
+      return nullptr;
+    }
+  return s;
+}
+
+void staging_give(Staging *s) {
+  if (!s) return;
+  {
+    std::lock_guard<std::mutex> lock(g_mu);
+    if (g_handles > 0 && g_nidle < kKeep) {
+      g_idle[g_nidle++] = s;
+      return;
+    }
+  }
+  destroy(s);
+}
+
+void staging_retain() {
+  std::lock_guard<std::mutex> lock(g_mu);
+  ++g_handles;
+}
+
+void staging_release() {
+  Staging *drop[kKeep];
+  int n = 0;
+  {
+    std::lock_guard<std::mutex> lock(g_mu);
+    if (--g_handles > 0) return;
+    while (g_nidle > 0) drop[n++] = g_idle[--g_nidle];
+  }
+  while (n > 0) destroy(drop[--n]);
+}
+
+void host_copy(void *dst, const void *src, size_t bytes) {
+  char *d = static_cast<char *>(dst);
+  const char *s = static_cast<const char *>(src);
+  std::thread th[kCopyThreads - 1];
+  size_t begin = 0;
+  int started = 0;
+  const size_t share = bytes / kCopyThreads / 4096 * 4096;
+  if (share >= kThreadBytes) {
+    try {
+      for (; started < kCopyThreads - 1; ++started) {
+        const size_t b = begin;
+        th[started] = std::thread([d, s, b, share] { std::memcpy(d + b, s + b, share); });
+        begin += share;
+      }
+    } catch (const std::system_error &) {  // no thread to be had: the rest here
+    }
+  }
+  std::memcpy(d + begin, s + begin, bytes - begin);
+  for (int t = 0; t < started; ++t) th[t].join();
+}
+
+}  // namespace oll

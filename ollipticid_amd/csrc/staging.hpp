@@ -1,0 +1,33 @@
+// Pinned host buffers that calls exchanging arrays with the host borrow.
+//
+// A call takes one Staging for itself and returns it; kernels read and write
+// the buffers over PCIe while the host copies the other half.  At most
+// kKeep idle ones are kept, and none once no handle (hierarchy or engine) is
+// left.  Any thread may take one: a Staging has one user at a time and no
+// tie to a device or stream.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cstddef>
+
+namespace oll {
+
+struct Staging {
+  static constexpr size_t kBytes = size_t(4) << 20;  // per half
+  char *half[2] = {nullptr, nullptr};
+};
+
+// null when the memory cannot be had
+Staging *staging_take();
+void staging_give(Staging *s);
+// a handle begins or ends
+void staging_retain();
+void staging_release();
+
+// copies of several megabytes by up to kCopyThreads threads: a copy into
+// fresh pages is bound by the faults of one thread (204 MB: 43 or 14.7 ms
+// with one thread, 4 KiB or 2 MiB pages, 17.2 or 6.1 with four)
+void host_copy(void *dst, const void *src, size_t bytes);
+
+}  // namespace oll

@@ -48,3 +48,46 @@ def test_coarsest_solve(eq, n):
         for ib in range(s.nbox):
             assert rel_err(h.get_field(ib, oa.F_U), s.field(ib, O.F_U)) < 1e-12, ib
     h.close()
+
+
+@pytest.mark.parametrize("n,order", [(25, 2), (33, 8), (65, 4), (81, 6), (129, 2)])
+def test_field_exchange(n, order):
+    """A field written and read back whole, in one piece and in several (a
+    half of the pinned staging holds 2^19 points), and single points of it
+    through the interpolation at grid points."""
+    h = oa.Hierarchy(oa.problem_from_argv(argv(0, n, order)))
+    rng = np.random.default_rng(7)
+    for ib in (h.nbox - 1, h.nbox - 2):
+        b = h.boxes()[ib]
+        a = rng.standard_normal(b["n"][::-1])
+        h.set_field(ib, oa.F_V, a)
+        assert np.array_equal(h.get_field(ib, oa.F_V), a)
+        ijk = np.stack([rng.integers(1, b["n"][a_] - 1, 500) for a_ in range(3)], axis=1)
+        xyz = np.array(b["origin"]) + ijk * np.array(b["d"])
+        got = h.interp(oa.F_V, np.full(500, ib), xyz, 3)
+        assert np.array_equal(got, a[ijk[:, 2], ijk[:, 1], ijk[:, 0]])
+    h.close()
+
+
+@pytest.mark.parametrize("order", range(1, 10))
+def test_interp_orders(order):
+    """Every interpolation order against the oracle, bit for bit, on both
+    sides of each change of route (few points, one chunk, several)."""
+    h, s = pair(argv(0, 25, 4))
+    seed_state(h, s, 3)
+    ib = s.nbox - 1
+    b = h.boxes()[ib]
+    rng = np.random.default_rng(order)
+    lo, hi = np.array(b["origin"]), np.array(b["end"])
+    xyz = lo + (hi - lo) * rng.uniform(0.0, 1.0, (65537 + 1000, 3))
+    box = np.full(len(xyz), ib, dtype=np.int32)
+    few = h.interp(oa.F_U, box[:4096], xyz[:4096], order)
+    want = [s.interp(ib, O.F_U, O.I_LAGRANGE, order, *x) for x in xyz[:200]]
+    assert np.array_equal(few[:200], want)
+    for count in (1, 15, 17, 4097, 65536, 65537, len(xyz)):
+        got = h.interp(oa.F_U, box[:count], xyz[:count], order)
+        assert np.array_equal(got[:4096], few[:count])
+        # the last points alone take the short route
+        tail = min(count, 50)
+        assert np.array_equal(got[-tail:], h.interp(oa.F_U, box[:tail], xyz[count - tail:count], order))
+    h.close()
