@@ -549,6 +549,14 @@ int transfer_fields(Hier &H, hipStream_t s, int from, int ffield, int to, int tf
   for (int t = 0; t < nt; ++t) {
     const DevBox &B = H.hbox[size_t(ft + t)];
     const long long np = npts(B), plane = (long long)B.n[0] * B.n[1];
+    if (nodes > 2) {  // Lagrange: tiles
+      for (int k = 0; k < B.n[2]; k += kXferTile[2])
+        for (int j = 0; j < B.n[1]; j += kXferTile[1])
+          for (int i = 0; i < B.n[0]; i += kXferTile[0])
+            blocks.push_back(PtBlock{H.dbox + ft + t, dx + refs[size_t(t)].off, refs[size_t(t)].cnt,
+                                     mode, 0u, 0u, i, j, k});
+      continue;
+    }
     for (long long q0 = 0; q0 < np; q0 += kPtThreads)
       blocks.push_back(PtBlock{H.dbox + ft + t, dx + refs[size_t(t)].off, refs[size_t(t)].cnt, mode,
                                unsigned(q0), unsigned(std::min<long long>(kPtThreads, np - q0)),
@@ -606,12 +614,6 @@ void set_fused_sweeps(bool on) { g_fused_sweeps = on; }
 static bool g_shared_loads = true;
 void set_shared_loads(bool on) { g_shared_loads = on; }
 bool shared_loads() { return g_shared_loads; }
-// columns pay at orders 6 and 8 (3 and 4 points per column share 8^3 and
-// 10^3 node stencils: ghost fill of the N=161 6th-order workload 766 ->
-// 502 us per launch); at orders 2 and 4 the halved thread count and lower
-// occupancy cost more than the saved loads (4th-order binary: 10% slower
-// alone), so those fill point by point
-bool ghost_columns_for(int order) { return g_shared_loads && order >= 6; }
 bool fused_sweeps() { return g_fused_sweeps; }
 
 void Schedule::clear() {
@@ -1040,7 +1042,7 @@ struct Builder {
         nb += point_blocks(H, k - 1, false);
       if (kind == Launch::PROLONG) nb += point_blocks(H, k, false);
       if (kind == Launch::GHOST && !mg)
-        nb += point_blocks(H, k, true, ghost_columns_for(H.level_order(k)));
+        nb += point_blocks(H, k, true, shared_loads());
     }
     const int reps = block_reps(members, nb);
     for (size_t h = 0; h < M.size(); ++h) {
@@ -1063,14 +1065,14 @@ struct Builder {
       if (kind == Launch::PROLONG) points(H, k, k, H.pv, false, mg, groups[{0, 0}], false, reps);
       if (kind == Launch::GHOST && !mg)
         points(H, k, k, H.gf, true, 0, groups[{H.level_order(k), 0}],
-               ghost_columns_for(H.level_order(k)), reps);
+               shared_loads(), reps);
     }
     for (auto &g : groups) {
       if (g.second.empty()) continue;
       Launch L{kind};
       L.order = g.first.first;
       L.eq = g.first.second;
-      L.mode = kind == Launch::GHOST && ghost_columns_for(L.order) ? 1 : 0;
+      L.mode = kind == Launch::GHOST && shared_loads() ? 1 : 0;
       L.off = S.add(g.second);
       L.n = int(g.second.size());
       S.launches.push_back(L);

@@ -13,7 +13,7 @@
 //   k_restrict_u        elliptic.cc:1543-1546 (Transferir INSIDE LAGRANGE 3)
 //   k_restrict_defect   elliptic.cc:1625-1747 (W = S - R, restrict, S = W + R)
 //   k_prolong           elliptic.cc:1827-1902 (V = u - ww, LINEAR, u += V)
-//   k_ghost_fill        elliptic.cc:1905-1908 (BOUNDARY LAGRANGE order+1)
+//   k_ghost_fill, k_ghost_tiles  elliptic.cc:1905-1908 (BOUNDARY LAGRANGE order+1)
 //   k_coarse_solve      elliptic.cc:1782-1816 (coarsest-level loop)
 //   k_coefficients      operator.cc:752-868, 2193-2380 (b, c, d, e)
 //   k_adm_sphere        elliptic.cc:2447-2611 Compute_ADM_Mass
@@ -1605,6 +1605,194 @@ __device__ __forceinline__ double trilinear_field(ConstBox &S, const void *f, Co
 #undef V
 }
 
+// ------------------------------------------------------------------
+// Lagrange interpolation of a block of target points as one tensor product.
+// The targets nt[0] x nt[1] x nt[2] from t0 take one source box; per axis
+// each has its first node, node count (1 on a node) and weights (the
+// transfer tables).  The source nodes they read (their bounding box) are
+// staged in LDS; then the sums over z are formed for every (x, y) node and z
+// target, from these the sums over y for every (x node, y target, z target),
+// then those over x: tinterp's sums for every target, in its order and with
+// its roundings (the same bits), each formed once instead of by every target
+// that shares it: 3 KP instead of KP^3 products per target, times the few
+// extra nodes at a tile's edge.  Bound by the LDS reads of the products.
+// ------------------------------------------------------------------
+template <int KP>
+struct TileLds {
+  // node extents of 16 targets refined by two (16 / 2 + KP + 1) and of the
+  // ghost width along a face's normal (KP + 3); larger regions (targets
+  // coarser than the source) take the point-by-point path
+  static constexpr int S = 9 + KP, U = KP + 3;
+  static constexpr int kNodes = S * S * U > 256 * U ? S * S * U : 256 * U;
+  static constexpr int kZ = 16 * S * U;
+  double a[kNodes];  // nodes [z][y][x]; then sums over y [z target][y target][x]
+  double z[kZ];      // sums over z [z target][y][x]
+  double w[3][16 * KP];
+  int first[3][16];  // from the region's low corner
+  int cnt[3][16];
+  int lo[3], ext[3];
+};
+
+// writes field tf at every target for which want(i, j, k) holds and some
+// source holds the point: `bits` are the flags that make a source eligible
+// (bit 0 its non-ghost part, bit 1 its extent), the last eligible source
+// counts; to_zero: the last source alone decides, 0 where it is not eligible
+template <int KP, class W>
+__device__ __forceinline__ void tile_transfer(TileLds<KP> &L, const PtBlock &Bk, ConstBox &T,
+                                              const int t0[3], const int nt[3], unsigned bits, int ff,
+                                              int tf, bool to_zero, W &&want) {
+  ConstXfer *xs = (ConstXfer *)Bk.src;
+  // the tile's source: lanes 0-15, 16-31, 32-47 of every wave hold the
+  // targets of axes x, y, z
+  const int lane = int(threadIdx.x & 63u), la = lane >> 4, li = lane & 15;
+  const int lt0 = la == 0 ? t0[0] : (la == 1 ? t0[1] : t0[2]);
+  const int lnt = la == 0 ? nt[0] : (la == 1 ? nt[1] : (la == 2 ? nt[2] : 0));
+  const bool lv = li < lnt;
+  const unsigned long long vm = __ballot(lv);
+  int src = -1;
+  bool mixed = false;
+  unsigned lf = 0;
+  for (int x = Bk.nsrc - 1; x >= 0; --x) {
+    const unsigned char *fp = la == 0 ? xs[x].ax[0].flags : (la == 1 ? xs[x].ax[1].flags : xs[x].ax[2].flags);
+    lf = lv ? fp[lt0 + li] : 0u;
+    bool every = false, some = false;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      if (!(bits & (1u << q))) continue;
+      const unsigned long long m = __ballot((lf >> q) & 1u);
+      every = every || m == vm;
+      some = some || ((m & 0xffffull) && (m & 0xffff0000ull) && (m & 0xffff00000000ull));
+    }
+    if (every) {
+      src = x;
+      break;
+    }
+    mixed = some;
+    if (mixed || to_zero) break;
+  }
+  const int total = nt[0] * nt[1] * nt[2];
+  const float in0 = 1.0f / float(nt[0]), in1 = 1.0f / float(nt[1]);
+  if (!mixed && src < 0 && !to_zero) return;
+  bool fits = !mixed && src >= 0;
+  if (fits) {
+    ConstXfer &X = xs[src];
+    if (threadIdx.x < 64) {
+      int first = 1 << 28, cnt = 1;
+      if (lv) {
+        const bool on = (lf & 4u) != 0;
+        const int *p = la == 0 ? (on ? X.ax[0].coinc : X.ax[0].start)
+                               : (la == 1 ? (on ? X.ax[1].coinc : X.ax[1].start)
+                                          : (on ? X.ax[2].coinc : X.ax[2].start));
+        first = p[lt0 + li];
+        cnt = on ? 1 : KP;
+        const double *w = (la == 0 ? X.ax[0].w : (la == 1 ? X.ax[1].w : X.ax[2].w)) + (lt0 + li) * KP;
+#pragma unroll
+        for (int m = 0; m < KP; ++m) L.w[la][li * KP + m] = on ? 1.0 : w[m];
+      }
+      int lo = first, hi = lv ? first + cnt : 0;
+#pragma unroll
+      for (int d = 1; d < 16; d <<= 1) {
+        lo = min(lo, __shfl_xor(lo, d, 16));
+        hi = max(hi, __shfl_xor(hi, d, 16));
+      }
+      if (la < 3) {
+        L.first[la][li] = first - lo;
+        L.cnt[la][li] = cnt;
+        if (li == 0) {
+          L.lo[la] = lo;
+          L.ext[la] = hi - lo;
+        }
+      }
+    }
+    __syncthreads();
+    const int ex = L.ext[0], ey = L.ext[1], ez = L.ext[2];
+    fits = ex * ey * ez <= TileLds<KP>::kNodes && nt[2] * ey * ex <= TileLds<KP>::kZ &&
+           nt[2] * nt[1] * ex <= TileLds<KP>::kNodes;
+    if (fits) {
+      ConstBox &S = cbox(X.src);
+      const void *f = S.f[ff];
+      const int lx = L.lo[0], ly = L.lo[1], lz = L.lo[2];
+      const float ix = 1.0f / float(ex), iy = 1.0f / float(ey);
+      for (int q = threadIdx.x; q < ex * ey * ez; q += kPtThreads) {
+        const int r = int(fast_div(unsigned(q), unsigned(ex), ix)), x = q - r * ex;
+        const int z = int(fast_div(unsigned(r), unsigned(ey), iy)), y = r - z * ey;
+        L.a[q] = ld<double>(f, boff(S, lx + x, ly + y, lz + z));
+      }
+      __syncthreads();
+      const int exy = ex * ey;
+      for (int q = threadIdx.x; q < nt[2] * exy; q += kPtThreads) {
+        const int zt = int(fast_div(unsigned(q), unsigned(exy), ix * iy)), r = q - zt * exy;
+        const double *v = L.a + L.first[2][zt] * exy + r, *w = L.w[2] + zt * KP;
+        const int n = L.cnt[2][zt];
+        double uk = 0.0;
+        if (n == 1) {
+          uk += v[0] * w[0];
+        } else {
+#pragma unroll
+          for (int K = 0; K < KP; ++K) uk += v[K * exy] * w[K];
+        }
+        L.z[q] = uk;
+      }
+      __syncthreads();
+      for (int q = threadIdx.x; q < nt[2] * nt[1] * ex; q += kPtThreads) {
+        const int r = int(fast_div(unsigned(q), unsigned(ex), ix)), x = q - r * ex;
+        const int zt = int(fast_div(unsigned(r), unsigned(nt[1]), in1)), yt = r - zt * nt[1];
+        const double *v = L.z + zt * exy + L.first[1][yt] * ex + x, *w = L.w[1] + yt * KP;
+        const int n = L.cnt[1][yt];
+        double uj = 0.0;
+        if (n == 1) {
+          uj += v[0] * w[0];
+        } else {
+#pragma unroll
+          for (int J = 0; J < KP; ++J) uj += v[J * ex] * w[J];
+        }
+        L.a[q] = uj;
+      }
+      __syncthreads();
+      for (int q = threadIdx.x; q < total; q += kPtThreads) {
+        const int r = int(fast_div(unsigned(q), unsigned(nt[0]), in0)), xt = q - r * nt[0];
+        const int zt = int(fast_div(unsigned(r), unsigned(nt[1]), in1)), yt = r - zt * nt[1];
+        const int i = t0[0] + xt, j = t0[1] + yt, k = t0[2] + zt;
+        if (!want(i, j, k)) continue;
+        const double *v = L.a + r * ex + L.first[0][xt], *w = L.w[0] + xt * KP;
+        const int n = L.cnt[0][xt];
+        double acc = 0.0;
+        if (n == 1) {
+          acc += v[0] * w[0];
+        } else {
+#pragma unroll
+          for (int I = 0; I < KP; ++I) acc += v[I] * w[I];
+        }
+        st<double>(T.f[tf], boff(T, i, j, k), acc);
+      }
+      return;
+    }
+  }
+  // sources that differ over the tile, or a region beyond the LDS: point by
+  // point
+#pragma unroll 1
+  for (int q = threadIdx.x; q < total; q += kPtThreads) {
+    const int r = int(fast_div(unsigned(q), unsigned(nt[0]), in0)), xt = q - r * nt[0];
+    const int zt = int(fast_div(unsigned(r), unsigned(nt[1]), in1)), yt = r - zt * nt[1];
+    const int t[3] = {t0[0] + xt, t0[1] + yt, t0[2] + zt};
+    if (!want(t[0], t[1], t[2])) continue;
+    const unsigned o = boff(T, t[0], t[1], t[2]);
+    for (int x = Bk.nsrc - 1; x >= 0; --x) {
+      ConstXfer &X = xs[x];
+      unsigned fl[3];
+      if (axis_flags(X, t, fl) & bits) {
+        ConstBox &S = cbox(X.src);
+        st<double>(T.f[tf], o, tinterp<KP>(S, S.f[ff], X, t, fl));
+        break;
+      }
+      if (to_zero) {
+        st<double>(T.f[tf], o, 0.0);
+        break;
+      }
+    }
+  }
+}
+
 // multigrid::Transferir (multigrid.cc:122-141, ffunction.cc:2436-2475):
 // every point of the region (PtBlock::mg bits 0-1: 0 all, 1 interior, 2
 // ghost shell) of the listed target boxes takes field ff of the source
@@ -1613,8 +1801,10 @@ __device__ __forceinline__ double trilinear_field(ConstBox &S, const void *f, Co
 // (or, with `all` (bit 2), whose extent does); with `to_zero` (bit 3) the
 // last source alone decides and a point it does not hold is set to 0 (the
 // reference's source loop overwrites every point on each pass)
-template <int KP>
-__global__ __launch_bounds__(kPtThreads) void k_transfer_fields(const PtBlock *__restrict__ blocks,
+// Linear transfers go point by point, Lagrange ones by tiles of
+// kXferTile targets (tile_transfer): N=129 8th order, one 135^3 box from its
+// parent, 1175 -> 78 us.
+__global__ __launch_bounds__(kPtThreads) void k_transfer_linear(const PtBlock *__restrict__ blocks,
                                                                 int ff, int tf) {
   const PtBlock Bk = blocks[xcd_block()];
   ConstBox &T = cbox(Bk.box);
@@ -1634,14 +1824,10 @@ __global__ __launch_bounds__(kPtThreads) void k_transfer_fields(const PtBlock *_
       if ((f & 1) || (all && (f & 2))) {
         ConstBox &S = cbox(X.src);
         double v;
-        if constexpr (KP == 2) {
-          if (f & 4)  // a source node: its value (interpolation.cc:140-147)
-            v = ld<double>(S.f[ff], boff(S, X.ax[0].coinc[i], X.ax[1].coinc[j], X.ax[2].coinc[k]));
-          else
-            v = trilinear_field(S, S.f[ff], X, t);
-        } else {
-          v = tinterp<KP>(S, S.f[ff], X, t, fl);
-        }
+        if (f & 4)  // a source node: its value (interpolation.cc:140-147)
+          v = ld<double>(S.f[ff], boff(S, X.ax[0].coinc[i], X.ax[1].coinc[j], X.ax[2].coinc[k]));
+        else
+          v = trilinear_field(S, S.f[ff], X, t);
         st<double>(T.f[tf], o, v);
         return;
       }
@@ -1650,6 +1836,25 @@ __global__ __launch_bounds__(kPtThreads) void k_transfer_fields(const PtBlock *_
         return;
       }
     }
+  });
+}
+
+template <int KP>
+__global__ __launch_bounds__(kPtThreads) void k_transfer_tiles(const PtBlock *__restrict__ blocks,
+                                                               int ff, int tf) {
+  __shared__ TileLds<KP> L;
+  const PtBlock Bk = blocks[xcd_block()];
+  ConstBox &T = cbox(Bk.box);
+  const int t0[3] = {Bk.i0, Bk.j0, Bk.k0};
+  const int nt[3] = {min(kXferTile[0], T.n[0] - t0[0]), min(kXferTile[1], T.n[1] - t0[1]),
+                     min(kXferTile[2], T.n[2] - t0[2])};
+  const int region = Bk.mg & 3, all = (Bk.mg >> 2) & 1, to_zero = (Bk.mg >> 3) & 1;
+  // a tile of interior points has none of the ghost shell
+  if (region == 2 && is_interior(T, t0[0], t0[1], t0[2]) &&
+      is_interior(T, t0[0] + nt[0] - 1, t0[1] + nt[1] - 1, t0[2] + nt[2] - 1))
+    return;
+  tile_transfer<KP>(L, Bk, T, t0, nt, all ? 3u : 1u, ff, tf, to_zero, [&](int i, int j, int k) {
+    return region == 0 || is_interior(T, i, j, k) == (region == 1);
   });
 }
 
@@ -1993,6 +2198,41 @@ __device__ __forceinline__ bool shell_column(ConstBox &B, unsigned q, int &i, in
   return true;
 }
 
+// the targets of the kColSuper^2 column slots from slot q (a multiple of
+// them): first point and extent of the tile, R points along the normal
+__device__ __forceinline__ void shell_tile(ConstBox &B, unsigned q, int t0[3], int nt[3]) {
+  constexpr unsigned kSlots = kColSuper * kColSuper;
+  const unsigned R = unsigned(B.R);
+  const unsigned n0 = unsigned(B.n[0]), n1 = unsigned(B.n[1]), n2 = unsigned(B.n[2]);
+  const unsigned zc = face_slots(n0, n1), yc = face_slots(n0, n2 - 2 * R);
+  int axis;
+  unsigned f0, f1, side;  // the face's extents, its side
+  if (q < 2 * zc) {
+    axis = 2; f0 = n0; f1 = n1; side = q >= zc; q -= side * zc;
+  } else if ((q -= 2 * zc) < 2 * yc) {
+    axis = 1; f0 = n0; f1 = n2 - 2 * R; side = q >= yc; q -= side * yc;
+  } else {
+    q -= 2 * yc;
+    axis = 0; f0 = n1 - 2 * R; f1 = n2 - 2 * R;
+    const unsigned xc = face_slots(f0, f1);
+    side = q >= xc; q -= side * xc;
+  }
+  const unsigned tx = col_tiles(f0), tile = q / kSlots;
+  const unsigned ty = tile / tx;
+  const unsigned a0 = (tile - ty * tx) * kColSuper, a1 = ty * kColSuper;
+  const int e0 = int(min(unsigned(kColSuper), f0 - a0)), e1 = int(min(unsigned(kColSuper), f1 - a1));
+  const int nn = axis == 0 ? int(n0) : (axis == 1 ? int(n1) : int(n2));
+  const int edge = side ? nn - int(R) : 0, r = int(R);
+  // z faces (x, y), y faces (x, z), x faces (y, z); interior along the axes
+  // whose faces come before
+  t0[0] = axis == 0 ? edge : int(a0);
+  t0[1] = axis == 1 ? edge : (axis == 2 ? int(a1) : r + int(a0));
+  t0[2] = axis == 2 ? edge : r + int(a1);
+  nt[0] = axis == 0 ? r : e0;
+  nt[1] = axis == 1 ? r : (axis == 2 ? e1 : e0);
+  nt[2] = axis == 2 ? r : e1;
+}
+
 // ghost shell of refinement boxes from the coarser level (Lagrange
 // order+1, KP = order+2 nodes per axis); one thread per shell point,
 // point q being layer q mod R of column slot q / R (shell_column), so that
@@ -2022,365 +2262,23 @@ __global__ __launch_bounds__(kPtThreads) void k_ghost_fill(const PtBlock *__rest
   });
 }
 
-// Ghost shell of refinement boxes, one thread per shell column (above).
-// The column's points share the node ranges and weights of the two axes
-// across the slab, so the node values are loaded once for all of them over
-// the union of their node ranges along the normal (at most KP + 3 nodes);
-// each point's sums run over its own nodes in tinterp's order (z innermost,
-// then y, then x, ascending), so every value is tinterp's to the bit.
-// Columns whose points take different sources fall back to tinterp point
-// by point.
-// The nodes a column's fast path reads (the per-axis ranges below: the
-// two axes across the slab and the union along the normal) and its source;
-// false when the column takes the point-by-point fallback
-template <int KP, int ax>
-__device__ __forceinline__ bool column_region(const PtBlock &Bk, const int p0[3], int &src,
-                                              int lo3[3], int hi3[3]) {
-  constexpr int KU = KP + 3;
-  constexpr int RG = (KP - 2) / 2;
-  ConstXfer *xs = (ConstXfer *)Bk.src;
-  unsigned fn[RG], fl0[3] = {0, 0, 0};
-  src = -1;
-#pragma unroll
-  for (int l = 0; l < RG; ++l) {
-    int sl = -1;
-    fn[l] = 0;
-    int t[3] = {p0[0], p0[1], p0[2]};
-    t[ax] += l;
-    for (int x = Bk.nsrc - 1; x >= 0; --x) {
-      unsigned fl[3];
-      const unsigned f = axis_flags(xs[x], t, fl);
-      if (!(f & 3)) continue;
-      sl = x;
-      fn[l] = fl[ax];
-      if (l == 0) {
-        fl0[0] = fl[0];
-        fl0[1] = fl[1];
-        fl0[2] = fl[2];
-      }
-      break;
-    }
-    if (l == 0) src = sl;
-    if (sl < 0 || sl != src) return false;
-  }
-  ConstXfer &X = xs[src];
-#pragma unroll
-  for (int a = 0; a < 3; ++a) {
-    if (a == ax) continue;
-    lo3[a] = (fl0[a] & 4) ? X.ax[a].coinc[p0[a]] : X.ax[a].start[p0[a]];
-    hi3[a] = lo3[a] + ((fl0[a] & 4) ? 1 : KP);
-  }
-  int lo = 1 << 30, hi = -1;
-#pragma unroll
-  for (int l = 0; l < RG; ++l) {
-    const int t = p0[ax] + l;
-    const int first = (fn[l] & 4) ? X.ax[ax].coinc[t] : X.ax[ax].start[t];
-    lo = min(lo, first);
-    hi = max(hi, first + ((fn[l] & 4) ? 1 : KP) - 1);
-  }
-  if (hi - lo + 1 > KU) return false;
-  lo3[ax] = lo;
-  hi3[ax] = hi + 1;
-  return true;
-}
-
-// STAGED: the column's source nodes are read from lds, the workgroup's copy
-// of the source box's nodes [lb, lb + (nx, ny, ...)) (k_ghost_cols)
-template <int KP, int ax, bool STAGED>
-__device__ __forceinline__ void ghost_column(const PtBlock &Bk, ConstBox &T, const int p0[3],
-                                             const double *lds, const int lb[3], int nx, int ny) {
-  constexpr int KU = KP + 3;       // union of the column's node ranges, at most
-  constexpr int RG = (KP - 2) / 2;  // ghost width of the boxes of this stencil
-  ConstXfer *xs = (ConstXfer *)Bk.src;
-  int src[RG];
-  unsigned fn[RG];  // flags of the normal axis per point
-  unsigned fl0[3] = {0, 0, 0};
-  bool same = true;
-#pragma unroll
-  for (int l = 0; l < RG; ++l) {
-    src[l] = -1;
-    fn[l] = 0;
-    int t[3] = {p0[0], p0[1], p0[2]};
-    t[ax] += l;
-    for (int x = Bk.nsrc - 1; x >= 0; --x) {
-      unsigned fl[3];
-      const unsigned f = axis_flags(xs[x], t, fl);
-      if (!(f & 3)) continue;
-      src[l] = x;
-      fn[l] = fl[ax];
-      if (l == 0) {
-        fl0[0] = fl[0];
-        fl0[1] = fl[1];
-        fl0[2] = fl[2];
-      }
-      break;
-    }
-    same = same && src[l] == src[0];
-  }
-  if (src[0] < 0 || !same) {
-#pragma unroll
-    for (int l = 0; l < RG; ++l) {
-      if (src[l] < 0) continue;
-      int t[3] = {p0[0], p0[1], p0[2]};
-      t[ax] += l;
-      ConstXfer &X = xs[src[l]];
-      unsigned fl[3];
-      axis_flags(X, t, fl);
-      ConstBox &S = cbox(X.src);
-      st<double>(T.f[F_U], boff(T, t[0], t[1], t[2]), tinterp<KP>(S, S.f[F_U], X, t, fl));
-    }
-    return;
-  }
-  ConstXfer &X = xs[src[0]];
-  ConstBox &S = cbox(X.src);
-  const void *f = S.f[F_U];
-  // the two axes across the slab: shared nodes and weights (tinterp's)
-  int s0[3], kk[3];
-  const double *w[3];
-#pragma unroll
-  for (int a = 0; a < 3; ++a) {
-    if (fl0[a] & 4) {
-      s0[a] = X.ax[a].coinc[p0[a]];
-      kk[a] = 1;
-      w[a] = nullptr;
-    } else {
-      s0[a] = X.ax[a].start[p0[a]];
-      kk[a] = KP;
-      w[a] = X.ax[a].w + p0[a] * KP;
-    }
-  }
-  // the normal: each point's first node and count, their union from lo
-  int first[RG], cnt[RG];
-  int lo = 1 << 30, hi = -1;
-#pragma unroll
-  for (int l = 0; l < RG; ++l) {
-    const int t = p0[ax] + l;
-    if (fn[l] & 4) {
-      first[l] = X.ax[ax].coinc[t];
-      cnt[l] = 1;
-    } else {
-      first[l] = X.ax[ax].start[t];
-      cnt[l] = KP;
-    }
-    lo = min(lo, first[l]);
-    hi = max(hi, first[l] + cnt[l] - 1);
-  }
-  const int U = hi - lo + 1;
-  if (U > KU) {  // not a refinement by two along the normal: point by point
-#pragma unroll
-    for (int l = 0; l < RG; ++l) {
-      int t[3] = {p0[0], p0[1], p0[2]};
-      t[ax] += l;
-      unsigned fl[3];
-      axis_flags(X, t, fl);
-      st<double>(T.f[F_U], boff(T, t[0], t[1], t[2]), tinterp<KP>(S, f, X, t, fl));
-    }
-    return;
-  }
-  // each point's weights along the normal at union positions (zero outside
-  // its range, where no term is added)
-  double wn[RG][KU];
-#pragma unroll
-  for (int l = 0; l < RG; ++l) {
-    const int d = first[l] - lo;
-    const double *wl = (fn[l] & 4) ? nullptr : X.ax[ax].w + (p0[ax] + l) * KP;
-#pragma unroll
-    for (int u = 0; u < KU; ++u) {
-      double v = 0.0;
-      if (u >= d && u < d + cnt[l]) v = wl ? wl[u - d] : 1.0;
-      wn[l][u] = v;
-    }
-  }
-  s0[ax] = lo;
-  kk[ax] = U;
-  const Walk wk(S);
-  unsigned oI = boff(S, s0[0], s0[1], s0[2]);
-  unsigned cI = colourc(S, s0[0], s0[1], s0[2]);
-  unsigned rI = unsigned(s0[0]) - divc(S, unsigned(s0[0])) * wk.nc;
-  double acc[RG];
-#pragma unroll
-  for (int l = 0; l < RG; ++l) acc[l] = 0.0;
-  // a node of the union lies in point l's range
-#define OLL_IN(l, u) ((u) >= first[l] - lo && (u) < first[l] - lo + cnt[l])
-  for (int I = 0; I < kk[0]; ++I) {
-    double uj[RG];
-#pragma unroll
-    for (int l = 0; l < RG; ++l) uj[l] = 0.0;
-    double ujx = 0.0;  // normal along x: the shared (y, z) sum
-    unsigned oJ = oI, cJ = cI;
-    if (ax == 1) {
-      // normal along y: z sums of every union row, then per point over y
-      double uk[KU];
-#pragma unroll
-      for (int J = 0; J < KU; ++J) {
-        unsigned off = oJ, c = cJ;
-        double v[KP];
-#pragma unroll
-        for (int K = 0; K < KP; ++K) {
-          if constexpr (STAGED)
-            v[K] = (J < U && K < kk[2]) ? lds[((s0[2] + K - lb[2]) * ny + (s0[1] + J - lb[1])) * nx +
-                                              (s0[0] + I - lb[0])]
-                                        : 0.0;
-          else
-            v[K] = (J < U && K < kk[2]) ? ld<double>(f, off) : 0.0;
-          off += wk.z(c);
-        }
-        double s = 0.0;
-#pragma unroll
-        for (int K = 0; K < KP; ++K)
-          if (K < kk[2]) s += v[K] * (w[2] ? w[2][K] : 1.0);
-        uk[J] = s;
-        if (J < U) oJ += wk.y(cJ);
-      }
-#pragma unroll
-      for (int l = 0; l < RG; ++l)
-#pragma unroll
-        for (int J = 0; J < KU; ++J)
-          if (OLL_IN(l, J)) uj[l] += uk[J] * wn[l][J];
-    } else {
-      for (int J = 0; J < kk[1]; ++J) {
-        unsigned off = oJ, c = cJ;
-        const double wy = w[1] ? w[1][J] : 1.0;
-        if (ax == 2) {
-          // normal along z: one union row, then per point over z
-          double v[KU];
-#pragma unroll
-          for (int K = 0; K < KU; ++K) {
-            if constexpr (STAGED)
-              v[K] = K < U ? lds[((s0[2] + K - lb[2]) * ny + (s0[1] + J - lb[1])) * nx +
-                                 (s0[0] + I - lb[0])]
-                           : 0.0;
-            else
-              v[K] = K < U ? ld<double>(f, off) : 0.0;
-            off += wk.z(c);
-          }
-#pragma unroll
-          for (int l = 0; l < RG; ++l) {
-            double s = 0.0;
-#pragma unroll
-            for (int K = 0; K < KU; ++K)
-              if (OLL_IN(l, K)) s += v[K] * wn[l][K];
-            uj[l] += s * wy;
-          }
-        } else {
-          // normal along x: the shared row sum
-          double v[KP];
-#pragma unroll
-          for (int K = 0; K < KP; ++K) {
-            if constexpr (STAGED)
-              v[K] = K < kk[2] ? lds[((s0[2] + K - lb[2]) * ny + (s0[1] + J - lb[1])) * nx +
-                                     (s0[0] + I - lb[0])]
-                               : 0.0;
-            else
-              v[K] = K < kk[2] ? ld<double>(f, off) : 0.0;
-            off += wk.z(c);
-          }
-          double s = 0.0;
-#pragma unroll
-          for (int K = 0; K < KP; ++K)
-            if (K < kk[2]) s += v[K] * (w[2] ? w[2][K] : 1.0);
-          ujx += s * wy;
-        }
-        oJ += wk.y(cJ);
-      }
-    }
-    if (ax == 0) {
-#pragma unroll
-      for (int l = 0; l < RG; ++l)
-        if (OLL_IN(l, I)) {
-          double wI = 0.0;  // wn[l][I] without a dynamic register index
-#pragma unroll
-          for (int u = 0; u < KU; ++u)
-            if (u == I) wI = wn[l][u];
-          acc[l] += ujx * wI;
-        }
-    } else {
-      const double wx = w[0] ? w[0][I] : 1.0;
-#pragma unroll
-      for (int l = 0; l < RG; ++l) acc[l] += uj[l] * wx;
-    }
-    oI += wk.x(cI, rI);
-  }
-#undef OLL_IN
-#pragma unroll
-  for (int l = 0; l < RG; ++l) {
-    int t[3] = {p0[0], p0[1], p0[2]};
-    t[ax] += l;
-    st<double>(T.f[F_U], boff(T, t[0], t[1], t[2]), acc[l]);
-  }
-}
-
-// A workgroup takes one kColSuper^2 tile of a face's columns; when the
-// columns on the fast path share their source, the nodes they read (their
-// bounding box, at most kGhostLds) are staged in LDS once and every column
-// reads its stencil from there.  The same values in the same order either
-// way.
-constexpr int kGhostLds = 4608;
+// Ghost shell of refinement boxes by tiles: a workgroup takes kColSuper^2
+// columns of one face side (one block of slots, shell_column), R points
+// each, and interpolates them as one tensor product (tile_interp).  Point by
+// point (or column by column) every target summed its own (order + 2)^3
+// nodes.  Measured, per launch: N=129 8th order 400 -> 32 us, N=161 6th
+// order 322 -> 48, 16 x N=65 4th order 146 -> 36.
 template <int KP>
-__global__ __launch_bounds__(kPtThreads) void k_ghost_cols(const PtBlock *__restrict__ blocks) {
-  __shared__ double lds[kGhostLds];
-  __shared__ int red[9];  // lo[3], hi[3], min and max source, a column off the fast path
+__global__ __launch_bounds__(kPtThreads) void k_ghost_tiles(const PtBlock *__restrict__ blocks) {
+  __shared__ TileLds<KP> L;
   const PtBlock Bk = blocks[xcd_block()];
   ConstBox &T = cbox(Bk.box);
-  ConstXfer *xs = (ConstXfer *)Bk.src;
-  // every thread walks the same chunks: the barriers below are uniform
-  for (unsigned base = 0; base < Bk.nq; base += kPtThreads) {
-    int p0[3] = {0, 0, 0}, ax = 0;
-    const bool valid =
-        base + threadIdx.x < Bk.nq && shell_column(T, Bk.q0 + base + threadIdx.x, p0[0], p0[1], p0[2], ax);
-    int src = -1, lo3[3] = {0, 0, 0}, hi3[3] = {0, 0, 0};
-    bool fast = false;
-    if (valid) {
-      if (ax == 0)
-        fast = column_region<KP, 0>(Bk, p0, src, lo3, hi3);
-      else if (ax == 1)
-        fast = column_region<KP, 1>(Bk, p0, src, lo3, hi3);
-      else
-        fast = column_region<KP, 2>(Bk, p0, src, lo3, hi3);
-    }
-    if (threadIdx.x < 9) red[threadIdx.x] = threadIdx.x < 3 ? (1 << 30) : (threadIdx.x == 6 ? (1 << 30) : -1);
-    __syncthreads();
-    if (fast) {
-#pragma unroll
-      for (int a = 0; a < 3; ++a) {
-        atomicMin(&red[a], lo3[a]);
-        atomicMax(&red[3 + a], hi3[a]);
-      }
-      atomicMin(&red[6], src);
-      atomicMax(&red[7], src);
-    }
-    __syncthreads();
-    const int lb[3] = {red[0], red[1], red[2]};
-    const int nx = red[3] - red[0], ny = red[4] - red[1], nz = red[5] - red[2];
-    const bool staged = red[6] == red[7] && nx > 0 && ny > 0 && nz > 0 && nx * ny * nz <= kGhostLds;
-    if (staged) {
-      ConstBox &S = cbox(xs[red[6]].src);
-      const void *f = S.f[F_U];
-      const int nxy = nx * ny;
-      for (int q = threadIdx.x; q < nxy * nz; q += kPtThreads) {
-        const int z = q / nxy, r = q - z * nxy, y = r / nx, x = r - y * nx;
-        lds[q] = ld<double>(f, boff(S, lb[0] + x, lb[1] + y, lb[2] + z));
-      }
-    }
-    __syncthreads();
-    if (valid) {
-      if (staged && fast) {
-        if (ax == 0)
-          ghost_column<KP, 0, true>(Bk, T, p0, lds, lb, nx, ny);
-        else if (ax == 1)
-          ghost_column<KP, 1, true>(Bk, T, p0, lds, lb, nx, ny);
-        else
-          ghost_column<KP, 2, true>(Bk, T, p0, lds, lb, nx, ny);
-      } else {
-        if (ax == 0)
-          ghost_column<KP, 0, false>(Bk, T, p0, nullptr, lb, 0, 0);
-        else if (ax == 1)
-          ghost_column<KP, 1, false>(Bk, T, p0, nullptr, lb, 0, 0);
-        else
-          ghost_column<KP, 2, false>(Bk, T, p0, nullptr, lb, 0, 0);
-      }
-    }
-    __syncthreads();  // lds and red are reused by the next chunk
+  constexpr unsigned kSlots = kColSuper * kColSuper;
+  for (unsigned base = 0; base < Bk.nq; base += kSlots) {
+    int t0[3], nt[3];
+    shell_tile(T, Bk.q0 + base, t0, nt);
+    tile_transfer<KP>(L, Bk, T, t0, nt, 3u, F_U, F_U, false, [&](int, int, int) { return true; });
+    __syncthreads();  // L is reused by the next tile
   }
 }
 
@@ -3399,7 +3297,7 @@ void launch_prolong(hipStream_t s, const PtBlock *blocks, int nblocks) {
 template <int KP>
 void ghost_impl(hipStream_t s, const PtBlock *blocks, int nblocks, int columns) {
   if (columns)
-    hipLaunchKernelGGL(k_ghost_cols<KP>, dim3(nblocks), dim3(kPtThreads), 0, s, blocks);
+    hipLaunchKernelGGL(k_ghost_tiles<KP>, dim3(nblocks), dim3(kPtThreads), 0, s, blocks);
   else
     hipLaunchKernelGGL(k_ghost_fill<KP>, dim3(nblocks), dim3(kPtThreads), 0, s, blocks);
 }
@@ -3448,9 +3346,11 @@ bool launch_coarse_solve(hipStream_t s, const CoarseItem *items, int n, int max_
 bool launch_transfer_fields(hipStream_t s, const PtBlock *blocks, int nblocks, int ff, int tf,
                             int nodes) {
   if (nblocks == 0) return true;
-#define OLL_TF(KP) hipLaunchKernelGGL(k_transfer_fields<KP>, dim3(nblocks), dim3(kPtThreads), 0, s, blocks, ff, tf)
+#define OLL_TF(KP) hipLaunchKernelGGL(k_transfer_tiles<KP>, dim3(nblocks), dim3(kPtThreads), 0, s, blocks, ff, tf)
   switch (nodes) {
-    case 2: OLL_TF(2); break;
+    case 2:
+      hipLaunchKernelGGL(k_transfer_linear, dim3(nblocks), dim3(kPtThreads), 0, s, blocks, ff, tf);
+      break;
     case 3: OLL_TF(3); break;
     case 4: OLL_TF(4); break;
     case 5: OLL_TF(5); break;

@@ -7,7 +7,8 @@ import pytest
 
 import ollipticid_amd as oa
 from oracle import oracle as O
-from tests.test_gpu_parity import PUNC, pair, rel_err, seed_state
+from ollipticid_amd import native
+from tests.test_gpu_parity import CASES, PUNC, pair, rel_err, seed_state
 
 pytestmark = pytest.mark.gpu
 
@@ -90,4 +91,51 @@ def test_interp_orders(order):
         # the last points alone take the short route
         tail = min(count, 50)
         assert np.array_equal(got[-tail:], h.interp(oa.F_U, box[:tail], xyz[count - tail:count], order))
+    h.close()
+
+
+@pytest.mark.parametrize("case", ["o4_merge", "sf_o6", "o8", "o2_flip"])
+def test_ghost_tiles_equal_points(case):
+    """The ghost shells filled by tiles are those filled point by point, bit
+    for bit: every order, merged boxes, tiles cut by the faces' edges."""
+    out = []
+    for on in (False, True):
+        h = oa.Hierarchy(oa.problem_from_argv(CASES[case]))
+        try:
+            native.set_shared_loads(on)
+            rng = np.random.default_rng(9)
+            for ib, b in enumerate(h.boxes()):
+                h.set_field(ib, oa.F_U, 1e-2 * rng.standard_normal(b["n"][::-1]))
+            for lv in range(1, h.levels):
+                h.fas(lv)
+            out.append([h.get_field(ib, oa.F_U) for ib in range(h.nbox)])
+        finally:
+            native.set_shared_loads(True)
+            h.close()
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("order", range(2, 10))
+@pytest.mark.parametrize("case", ["o4_merge", "o2_flip"])
+def test_transfer_tiles(case, order):
+    """Lagrange transfers against the oracle at every target point: to a
+    finer level (one source box and several), to a coarser one and within a
+    level, over each region, with and without `all` and `to_zero`."""
+    h, s = pair(CASES[case])
+    seed_state(h, s, order)
+    rng = np.random.default_rng(order)
+    top = s.levels - 1
+    for frm, to in ((top - 1, top), (top, top - 1), (top - 2, top), (top, top)):
+        for region in (0, 1, 2):
+            for all_, to_zero in ((True, False), (False, False), (False, True)):
+                for ib in s.level_boxes(to):
+                    v = rng.standard_normal(s.field(ib, O.F_V).shape)
+                    s.field(ib, O.F_V)[:] = v
+                    h.set_field(ib, oa.F_V, v)
+                h.transfer(frm, oa.F_U, to, oa.F_V, region, 1, order, all_, to_zero)
+                s.transfer(frm, O.F_U, to, O.F_V, region, 1, order, int(all_), int(to_zero))
+                for ib in s.level_boxes(to):
+                    g, o = h.get_field(ib, oa.F_V), s.field(ib, O.F_V)
+                    assert rel_err(g, o) < 1e-12, (frm, to, region, all_, to_zero, ib)
     h.close()
