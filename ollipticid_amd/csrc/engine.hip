@@ -644,6 +644,9 @@ struct Builder {
     return ((B.n[0] - 2 * B.R + B.nc - 1) / B.nc + pts - 1) / pts;
   }
 
+  // threads for the slots of one colour row of B
+  static int slot_threads(const DevBox &B, int pts) { return (B.rl + pts - 1) / pts; }
+
   // threads per row of a level: colour points per interior row (colour
   // passes) or slots per colour row (whole-row kernels)
   // (pts: colour points a thread takes)
@@ -652,7 +655,7 @@ struct Builder {
     int m = 0;
     for (int b = f; b < f + n; ++b) {
       const DevBox &B = H.hbox[size_t(b)];
-      m = std::max(m, subrows ? B.rl : row_threads(B, pts));
+      m = std::max(m, subrows ? slot_threads(B, pts) : row_threads(B, pts));
     }
     return m;
   }
@@ -669,7 +672,7 @@ struct Builder {
     const int f = H.geo.level_first[size_t(level)], n = H.geo.level_count[size_t(level)];
     for (int b = f; b < f + n; ++b) {
       const DevBox &B = H.hbox[size_t(b)];
-      const int len = subrows ? B.rl : row_threads(B, pts);
+      const int len = subrows ? slot_threads(B, pts) : row_threads(B, pts);
       const int nseg = (len + seg - 1) / seg;
       const int rows = interior_rows(B) * (subrows ? B.nc : 1) * nseg;
       for (int r0 = 0; r0 < rows; r0 += rpb)
@@ -679,14 +682,14 @@ struct Builder {
 
   // blocks row_blocks() gives at reps = 1
   static long long row_block_count(const Hier &H, int level, bool subrows, int pr,
-                                   int threads = kRowThreads) {
+                                   int threads = kRowThreads, int pts = 1) {
     const int seg = std::min(pr, threads);
     const int rpb = std::max(1, threads / seg);
     const int f = H.geo.level_first[size_t(level)], n = H.geo.level_count[size_t(level)];
     long long nb = 0;
     for (int b = f; b < f + n; ++b) {
       const DevBox &B = H.hbox[size_t(b)];
-      const int len = subrows ? B.rl : row_threads(B, 1);
+      const int len = subrows ? slot_threads(B, pts) : row_threads(B, pts);
       const long long rows = (long long)interior_rows(B) * (subrows ? B.nc : 1) * ((len + seg - 1) / seg);
       nb += (rows + rpb - 1) / rpb;
     }
@@ -749,7 +752,7 @@ struct Builder {
       const int pts = mixed ? 1 : sweep_points(eq);
       for (int h : g.second) {
         pc = std::max(pc, per_row(*M[size_t(h)], lv[size_t(h)], false, pts));
-        ps = std::max(ps, per_row(*M[size_t(h)], lv[size_t(h)], true));
+        ps = std::max(ps, per_row(*M[size_t(h)], lv[size_t(h)], true, sweep_points(eq)));
       }
       std::vector<RowBlock> cb, sb;
       double bytes[5] = {0, 0, 0, 0, 0};
@@ -768,14 +771,14 @@ struct Builder {
       int sreps = 1;
       if (mixed) {
         long long nsb = 0;
-        for (int h : g.second) nsb += row_block_count(*M[size_t(h)], lv[size_t(h)], true, ps);
+        for (int h : g.second) nsb += row_block_count(*M[size_t(h)], lv[size_t(h)], true, ps, kRowThreads, sweep_points(eq));
         sreps = block_reps(g.second.size(), nsb);
       }
       for (int h : g.second) {
         const Hier &H = *M[size_t(h)];
         const int l = lv[size_t(h)];
         row_blocks(H, l, mixed ? nullptr : slot(H, l), false, pc, cb, threads, 1, pts);
-        if (mixed) row_blocks(H, l, slot(H, l), true, ps, sb, kRowThreads, sreps);
+        if (mixed) row_blocks(H, l, slot(H, l), true, ps, sb, kRowThreads, sreps, sweep_points(eq));
         for (int b = 0; b < H.geo.level_count[size_t(l)]; ++b)
           boxes.insert(H.dbox + H.geo.level_first[size_t(l)] + b);
         // algorithmic bytes per updated point: FP64 reads u, b, c, rho
@@ -860,15 +863,17 @@ struct Builder {
       if (lv[h] >= 0) groups[{M[h]->level_order(lv[h]), M[h]->prob.eq}].push_back(int(h));
     for (auto &g : groups) {
       int ps = 0;
-      for (int h : g.second) ps = std::max(ps, per_row(*M[size_t(h)], lv[size_t(h)], true));
+      const int pts = sweep_points(g.first.second);
+      for (int h : g.second) ps = std::max(ps, per_row(*M[size_t(h)], lv[size_t(h)], true, pts));
       std::vector<RowBlock> blocks;
       long long nb = 0;
-      for (int h : g.second) nb += row_block_count(*M[size_t(h)], lv[size_t(h)], true, ps);
+      for (int h : g.second)
+        nb += row_block_count(*M[size_t(h)], lv[size_t(h)], true, ps, kRowThreads, pts);
       const int reps = block_reps(g.second.size(), nb);
       for (int h : g.second) {
         const Hier &H = *M[size_t(h)];
         row_blocks(H, lv[size_t(h)], with_norm ? H.slot(H.slot_scratch()) : nullptr, true, ps,
-                   blocks, kRowThreads, reps);
+                   blocks, kRowThreads, reps, pts);
       }
       Launch L{Launch::RESIDUAL};
       L.order = g.first.first;
@@ -989,6 +994,26 @@ struct Builder {
       }
   }
 
+  // tiles of the prolongation into level k of H (the interior points of a
+  // refinement level, every point of a multigrid one), reps of them along z
+  // a block; returns the number of blocks
+  static long long prolong_tiles(const Hier &H, int k, int mg, int reps, std::vector<PtBlock> *out) {
+    const int f = H.geo.level_first[size_t(k)], n = H.geo.level_count[size_t(k)];
+    const int dz = kProTile[2] * reps;
+    long long nb = 0;
+    for (int t = 0; t < n; ++t) {
+      const DevBox &B = H.hbox[size_t(f + t)];
+      const Hier::XRef r = H.pv[size_t(k)][size_t(t)];
+      const int g = mg ? 0 : B.R;
+      for (int z = g; z < B.n[2] - g; z += dz)
+        for (int y = g; y < B.n[1] - g; y += kProTile[1])
+          for (int x = g; x < B.n[0] - g; x += kProTile[0], ++nb)
+            if (out)
+              out->push_back(PtBlock{H.dbox + f + t, H.dxfer + r.off, r.cnt, mg, 0u, unsigned(dz), x, y, z});
+    }
+    return nb;
+  }
+
   // Blocks per kPtThreads points (or per workgroup of rows) for a launch
   // over one request; a launch over several requests gives each block reps
   // times that many, which the kernels' threads step through, so that its
@@ -1040,7 +1065,7 @@ struct Builder {
       ++members;
       if ((kind == Launch::RESTRICT_U || kind == Launch::RESTRICT_DEFECT) && mg)
         nb += point_blocks(H, k - 1, false);
-      if (kind == Launch::PROLONG) nb += point_blocks(H, k, false);
+      if (kind == Launch::PROLONG) nb += prolong_tiles(H, k, mg, 1, nullptr);
       if (kind == Launch::GHOST && !mg)
         nb += point_blocks(H, k, true, shared_loads());
     }
@@ -1062,7 +1087,7 @@ struct Builder {
         else
           segments(H, k - 1, k, H.rw, groups[{H.level_order(k - 1), H.prob.eq}], true);
       }
-      if (kind == Launch::PROLONG) points(H, k, k, H.pv, false, mg, groups[{0, 0}], false, reps);
+      if (kind == Launch::PROLONG) prolong_tiles(H, k, mg, reps, &groups[{0, 0}]);
       if (kind == Launch::GHOST && !mg)
         points(H, k, k, H.gf, true, 0, groups[{H.level_order(k), 0}],
                shared_loads(), reps);

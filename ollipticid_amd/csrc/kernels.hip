@@ -564,6 +564,33 @@ __device__ __forceinline__ void lap_pair(const void *u, unsigned o, const Nbr<OR
   }
 }
 
+// N(u) and dN/du of the pair at byte offset o (EQ without first derivatives)
+template <int ORD, int EQ>
+__device__ __forceinline__ void point_op_pair(ConstBox &B, const double *u, unsigned o,
+                                              const Nbr<ORD / 2 + 1> &nb, const double u0[2],
+                                              double N[2], double dN[2]) {
+  double lu[2], b[2], c[2], d[2] = {0.0, 0.0}, e[2] = {0.0, 0.0};
+  ld_pair(B.f[F_B], o, b[0], b[1]);
+  ld_pair(B.f[F_C], o, c[0], c[1]);
+  if constexpr (EQ == 1) {
+    ld_pair(B.f[F_D], o, d[0], d[1]);
+    ld_pair(B.f[F_E], o, e[0], e[1]);
+  }
+  lap_pair<ORD>(u, o, nb, u0[0], u0[1], B.idx2[0], B.idx2[1], B.idx2[2], lu);
+#pragma unroll
+  for (int q = 0; q < 2; ++q)
+    nonlinear<EQ>(lu[q], B.dulap, b[q], c[q] + u0[q], d[q], e[q], N[q], dN[q]);
+}
+
+// rho of the pair of points (i, j, k), (i + nc, j, k): +0 outside the rho box
+__device__ __forceinline__ void rho_pair(ConstBox &B, unsigned o, int i, int nc, int j, int k,
+                                         double rho[2]) {
+  rho[0] = rho[1] = 0.0;
+  if ((unsigned(j - B.rlo[1]) < unsigned(B.rhi[1] - B.rlo[1])) &
+      (unsigned(k - B.rlo[2]) < unsigned(B.rhi[2] - B.rlo[2])) & (i + nc >= B.rlo[0]) & (i < B.rhi[0]))
+    ld_pair(B.f[F_RHO], o, rho[0], rho[1]);
+}
+
 template <int ORD, int EQ>
 __device__ __forceinline__ void smooth_pairs(const RowBlock &Bk, ConstBox &B, unsigned per_row,
                                              float inv_per_row, int colour) {
@@ -594,29 +621,14 @@ __device__ __forceinline__ void smooth_pairs(const RowBlock &Bk, ConstBox &B, un
       const Nbr<NC> nb = box_offs<NC, 8>(B, col, first % NC);
       const unsigned o = p * 8u;
       double *u = B.f[F_U];
-      double rho[2] = {0.0, 0.0};
-      // rho is +0 outside the rho box: a pair that reaches into it is read
-      // whole
-      if ((unsigned(j - B.rlo[1]) < unsigned(B.rhi[1] - B.rlo[1])) &
-          (unsigned(k - B.rlo[2]) < unsigned(B.rhi[2] - B.rlo[2])) & (i + NC >= B.rlo[0]) &
-          (i < B.rhi[0]))
-        ld_pair(B.f[F_RHO], o, rho[0], rho[1]);
-      double u0[2], lu[2], b[2], c[2], d[2] = {0.0, 0.0}, e[2] = {0.0, 0.0};
+      double rho[2], u0[2], N[2], dN[2], un[2];
+      rho_pair(B, o, i, NC, j, k, rho);
       ld_pair(u, o, u0[0], u0[1]);
-      ld_pair(B.f[F_B], o, b[0], b[1]);
-      ld_pair(B.f[F_C], o, c[0], c[1]);
-      if constexpr (EQ == 1) {
-        ld_pair(B.f[F_D], o, d[0], d[1]);
-        ld_pair(B.f[F_E], o, e[0], e[1]);
-      }
-      lap_pair<ORD>(u, o, nb, u0[0], u0[1], B.idx2[0], B.idx2[1], B.idx2[2], lu);
-      double un[2];
+      point_op_pair<ORD, EQ>(B, u, o, nb, u0, N, dN);
 #pragma unroll
       for (int q = 0; q < 2; ++q) {
-        double N, dN;
-        nonlinear<EQ>(lu[q], B.dulap, b[q], c[q] + u0[q], d[q], e[q], N, dN);
-        const double res = N - rho[q];
-        un[q] = u0[q] - res / dN;
+        const double res = N[q] - rho[q];
+        un[q] = u0[q] - res / dN[q];
         if (q == 0 || two) {
           rmax = fmax(rmax, fabs(res));
           if (!(un[q] == un[q])) rmax = __longlong_as_double(0x7ff0000000000000LL);
@@ -772,6 +784,34 @@ __global__ __launch_bounds__(kFusedThreads) void k_smooth_fused(const TileBlock 
   wave_norm(T.norm, rmax, seen);
 }
 
+// whole-row kernels, two slots a thread: slots 2t and 2t + 1 of sub-row sr
+// (row_slot); ok[q]: the slot holds an interior point.  Loads of the other
+// slot stay inside the field (rows precede and follow every interior row)
+template <int R, int NC = R + 1>
+__device__ __forceinline__ bool row_pair(const RowBlock &Bk, ConstBox &B, unsigned per_row,
+                                         float inv_per_row, unsigned rpb, unsigned lr0, unsigned &p,
+                                         int &c, int &s, int &i, int &j, int &k, bool ok[2]) {
+  const unsigned lrl = fast_div(threadIdx.x, per_row, inv_per_row);
+  unsigned t = threadIdx.x - lrl * per_row;
+  const unsigned lr = lr0 + lrl;
+  if (lrl >= rpb || lr >= unsigned(Bk.rows)) return false;
+  unsigned sr = unsigned(Bk.row0) + lr;
+  if (Bk.nseg > 1) {
+    const unsigned seg = sr % unsigned(Bk.nseg);
+    sr /= unsigned(Bk.nseg);
+    t += seg * per_row;
+  }
+  const unsigned row = sr / NC;
+  c = int(sr - row * NC);
+  row_jk<R>(B, row, j, k);
+  s = int(unsigned(c + NC * 3 * kMaxAxisPoints - j - k) % NC);
+  i = s + int(2 * t) * NC;
+  ok[0] = i >= R && i < B.n[0] - R;
+  ok[1] = i + NC >= R && i + NC < B.n[0] - R;
+  p = unsigned(c) * unsigned(B.cs) + unsigned(k) * unsigned(B.ps) + unsigned(j) * unsigned(B.rs) + 2 * t;
+  return ok[0] || ok[1];
+}
+
 // operator on the interior: mode RES_OPERATOR r = N(u), RES_DEFECT
 // w = rho - N(u), RES_DERIVATIVE r = dN/du_p; the norm is max |N(u)|
 template <int ORD, int EQ>
@@ -784,6 +824,35 @@ __global__ __launch_bounds__(kRowThreads) void k_residual(const RowBlock *__rest
   ConstBox &B = cbox(Bk.box);
   const double seen = norm_seen(Bk.norm);
   double rmax = 0.0;
+  if constexpr (sweep_points(EQ) == 2) {
+    // two slots a thread, as the colour passes (one: N=161 6th order 234 us a
+    // launch, 16 x N=65 4th order 67; two: 188 and 53)
+    double *out = mode == RES_DEFECT ? B.f[F_W] : B.f[F_R];
+    for_rows(Bk, per_row, inv_per_row, [&](unsigned rpb, unsigned lr0) {
+      unsigned p;
+      int c, s, i, j, k;
+      bool ok[2];
+      if (!row_pair<R>(Bk, B, per_row, inv_per_row, rpb, lr0, p, c, s, i, j, k, ok)) return;
+      const Nbr<R + 1> nb = box_offs<R + 1, 8>(B, c, s);
+      const unsigned o = p * 8u;
+      const double *u = B.f[F_U];
+      double rho[2] = {0.0, 0.0}, u0[2], N[2], dN[2], v[2];
+      if (mode == RES_DEFECT) rho_pair(B, o, i, R + 1, j, k, rho);
+      ld_pair(u, o, u0[0], u0[1]);
+      point_op_pair<ORD, EQ>(B, u, o, nb, u0, N, dN);
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        v[q] = mode == RES_DEFECT ? rho[q] - N[q] : (mode == RES_DERIVATIVE ? dN[q] : N[q]);
+        if (ok[q]) rmax = nan_max(rmax, fabs(N[q]));
+      }
+      if (ok[0] && ok[1])
+        st_pair(out, o, v[0], v[1]);
+      else
+        st<double>(out, ok[0] ? o : o + 8u, ok[0] ? v[0] : v[1]);
+    });
+    wave_norm(Bk.norm, rmax, seen);
+    return;
+  }
   for_rows(Bk, per_row, inv_per_row, [&](unsigned rpb, unsigned lr0) {
     unsigned p;
     int c, s, i, j, k;
@@ -816,7 +885,7 @@ template <int ORD, int EQ>
 __global__ __launch_bounds__(kRowThreads) void k_defect32(const RowBlock *__restrict__ blocks,
                                                           unsigned per_row, float inv_per_row) {
   constexpr int R = ORD / 2;
-  constexpr int NC = colours_of(ORD, EQ);
+  constexpr int NC = R + 1;
   const RowBlock Bk = blocks[xcd_block()];
   ConstBox &B = cbox(Bk.box);
   const double seen = norm_seen(Bk.norm);
@@ -824,19 +893,26 @@ __global__ __launch_bounds__(kRowThreads) void k_defect32(const RowBlock *__rest
   for_rows(Bk, per_row, inv_per_row, [&](unsigned rpb, unsigned lr0) {
     unsigned p;
     int c, s, i, j, k;
-    if (!row_slot<R, NC>(Bk, B, per_row, inv_per_row, rpb, lr0, p, c, s, i, j, k)) return;
+    bool ok[2];
+    if (!row_pair<R>(Bk, B, per_row, inv_per_row, rpb, lr0, p, c, s, i, j, k, ok)) return;
     const Nbr<NC> nb = box_offs<NC, 8>(B, c, s);
-    const unsigned o = p * 8u, o4 = p * 4u;
+    const unsigned o = p * 8u;
     const double *u = B.f[F_U];
-    const double rho = rho_at(B, o, i, j, k);
-    double N, dN;
-    point_op<ORD, EQ>(B, u, o, nb, ld<double>(u, o), i, j, k, N, dN);
-    const double res = rho - N;
-    st<float>(B.g[G_R], o4, float(res));
-    st<float>(B.g[G_Q], o4, float(dN - B.dulap));
-    st<float>(B.g[G_E], o4, 0.0f);
-    rmax = nan_max(rmax, fabs(res));
-    if (!(res == res)) rmax = __longlong_as_double(0x7ff0000000000000LL);
+    double rho[2], u0[2], N[2], dN[2];
+    rho_pair(B, o, i, NC, j, k, rho);
+    ld_pair(u, o, u0[0], u0[1]);
+    point_op_pair<ORD, EQ>(B, u, o, nb, u0, N, dN);
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      if (!ok[q]) continue;
+      const unsigned o4 = (p + unsigned(q)) * 4u;
+      const double res = rho[q] - N[q];
+      st<float>(B.g[G_R], o4, float(res));
+      st<float>(B.g[G_Q], o4, float(dN[q] - B.dulap));
+      st<float>(B.g[G_E], o4, 0.0f);
+      rmax = nan_max(rmax, fabs(res));
+      if (!(res == res)) rmax = __longlong_as_double(0x7ff0000000000000LL);
+    }
   });
   wave_norm(Bk.norm, rmax, seen);
 }
@@ -875,9 +951,18 @@ __global__ __launch_bounds__(kRowThreads) void k_update32(const RowBlock *__rest
   for_rows(Bk, per_row, inv_per_row, [&](unsigned rpb, unsigned lr0) {
     unsigned p;
     int c, s, i, j, k;
-    if (!row_slot<R>(Bk, B, per_row, inv_per_row, rpb, lr0, p, c, s, i, j, k)) return;
+    bool ok[2];
+    if (!row_pair<R>(Bk, B, per_row, inv_per_row, rpb, lr0, p, c, s, i, j, k, ok)) return;
     double *u = B.f[F_U];
-    st<double>(u, p * 8u, ld<double>(u, p * 8u) + double(ld<float>(B.g[G_E], p * 4u)));
+    const unsigned o = p * 8u;
+    double u0, u1;
+    ld_pair(u, o, u0, u1);
+    u0 += double(ld<float>(B.g[G_E], p * 4u));
+    u1 += double(ld<float>(B.g[G_E], p * 4u + 4u));
+    if (ok[0] && ok[1])
+      st_pair(u, o, u0, u1);
+    else
+      st<double>(u, ok[0] ? o : o + 8u, ok[0] ? u0 : u1);
   });
 }
 
@@ -2078,37 +2163,183 @@ __global__ __launch_bounds__(kPtThreads) void k_corr_v(const PtBlock *__restrict
 }
 
 // prolongation of the coarse correction v (k_corr_v) and u += I v (all
-// points on multigrid levels, interior points on refinement levels)
+// points on multigrid levels, interior points on refinement levels).  A
+// block covers a column of kProTile tiles (nq planes from (i0, j0, k0)); the
+// coarse nodes a tile reads are staged in LDS and the interpolation along x
+// is formed once per coarse row, so that a fine point costs four LDS reads
+// and its own u instead of eight scattered coarse loads: per launch N=161 187
+// -> 88 us, 16 x N=65 95 -> 55.  Each value is trilinear_corr's or
+// trilinear_nested's to the bit (x first, then y, then z); tiles whose
+// points take different sources go point by point.
 __global__ __launch_bounds__(kPtThreads) void k_prolong(const PtBlock *__restrict__ blocks) {
+  constexpr int TX = kProTile[0], TY = kProTile[1], TZ = kProTile[2];
+  static_assert(TX == 64 && TY * TZ * TX == 4 * kPtThreads && TY == 4 && TZ == 4, "thread mapping");
+  constexpr int VX = TX / 2 + 4, VY = TY / 2 + 3, VZ = TZ / 2 + 3;
+  __shared__ double V[VX * VY * VZ];  // coarse nodes [z][y][x]
+  __shared__ double A[VZ * VY * TX];  // interpolated along x [z][y][x target]
+  // per target of an axis (x, then y, then z): first node, node of a
+  // coincident target (-1: none), weights of the first and second node
+  constexpr int NT = TX + TY + TZ;
+  __shared__ int first[NT], same[NT];
+  __shared__ double wi[NT], wf[NT];
+  __shared__ int lo[3], ext[3];
   const PtBlock Bk = blocks[xcd_block()];
   ConstBox &T = cbox(Bk.box);
-  for_points(Bk, [&](unsigned off) {
-    int i, j, k;
-    pt_lex(Bk, T, off, i, j, k);
-    if (!Bk.mg && !is_interior(T, i, j, k)) return;
-    const int t[3] = {i, j, k};
-    // the target value is loaded first; its latency overlaps the source's
-    const unsigned o = boff(T, i, j, k);
-    const double u0 = ld<double>(T.f[F_U], o);
-    ConstXfer *xs = (ConstXfer *)Bk.src;
-    for (int x = Bk.nsrc - 1; x >= 0; --x) {
-      ConstXfer &X = xs[x];
-      unsigned fl[3];
-      const unsigned f = axis_flags(X, t, fl);
-      if (!(f & 3)) continue;  // all = true
-      ConstBox &S = cbox(X.src);
-      double v;
-      if (f & 4) {
-        v = ld<double>(S.f[F_V], boff(S, X.ax[0].coinc[i], X.ax[1].coinc[j], X.ax[2].coinc[k]));
-      } else if (X.affine) {
-        v = trilinear_nested(S, X, t);
-      } else {
-        v = trilinear_corr(S, X, t);
+  ConstXfer *xs = (ConstXfer *)Bk.src;
+  const int lane = int(threadIdx.x & 63u), wave = int(threadIdx.x >> 6);
+  const int g = Bk.mg ? 0 : T.R;  // the points taken: [g, n - g) on every axis
+  const int kend = min(Bk.k0 + int(Bk.nq), T.n[2] - g);
+  const int nx = min(TX, T.n[0] - g - Bk.i0), ny = min(TY, T.n[1] - g - Bk.j0);
+  for (int k0 = Bk.k0; k0 < kend; k0 += TZ) {
+    const int nz = min(TZ, kend - k0);
+    // the thread's four targets: (lane, wave, q); their u is loaded first
+    const int i = Bk.i0 + lane, j = Bk.j0 + wave;
+    const bool mine = lane < nx && wave < ny;
+    unsigned o[TZ];
+    double u0[TZ];
+#pragma unroll
+    for (int q = 0; q < TZ; ++q) {
+      o[q] = 0;
+      u0[q] = 0.0;
+      if (mine && q < nz) {
+        o[q] = boff(T, i, j, k0 + q);
+        u0[q] = ld<double>(T.f[F_U], o[q]);
       }
-      st<double>(T.f[F_U], o, u0 + v);
-      return;
     }
-  });
+    // the tile's source: lane x of every wave holds x target x; lanes 0-3 y
+    // and 4-7 z targets
+    const bool vx = lane < nx;
+    const bool vyz = lane < 4 ? lane < ny : (lane < 8 && lane - 4 < nz);
+    const int tyz = lane < 4 ? Bk.j0 + lane : k0 + (lane - 4);
+    const unsigned long long mx = __ballot(vx), myz = __ballot(vyz);
+    int src = -1;
+    bool mixed = false;
+    unsigned fx = 0, fyz = 0;
+    for (int x = Bk.nsrc - 1; x >= 0; --x) {
+      fx = vx ? xs[x].ax[0].flags[i] : 0u;
+      fyz = vyz ? (lane < 4 ? xs[x].ax[1].flags : xs[x].ax[2].flags)[tyz] : 0u;
+      bool every = false, some = false;
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const unsigned long long bx = __ballot((fx >> q) & 1u), byz = __ballot((fyz >> q) & 1u);
+        every = every || (bx == mx && byz == myz);
+        some = some || (bx && (byz & 0xfull) && (byz & 0xf0ull));
+      }
+      if (every) {
+        src = x;
+        break;
+      }
+      if ((mixed = some)) break;
+    }
+    bool fits = !mixed && src >= 0;
+    if (fits) {
+      ConstXfer &X = xs[src];
+      ConstBox &S = cbox(X.src);
+      // wave 0: the x targets; wave 1: y and z
+      if (wave < 2) {
+        const int ax = wave == 0 ? 0 : (lane < 4 ? 1 : 2);
+        const bool v = wave == 0 ? vx : vyz;
+        const int t = wave == 0 ? i : tyz;
+        const unsigned fl = wave == 0 ? fx : fyz;
+        const int slot = wave == 0 ? lane : TX + (lane < 4 ? lane : TY + (lane - 4));
+        int c = 1 << 28, cc = -1;
+        if (v) {
+          double a, b;
+          if (X.affine) {
+            const int q = t + (ax == 0 ? X.aff[0] : (ax == 1 ? X.aff[1] : X.aff[2]));
+            const int sn = ax == 0 ? S.n[0] : (ax == 1 ? S.n[1] : S.n[2]);
+            const bool mid = (q & 1) != 0;
+            c = q >> 1;
+            a = mid ? 0.5 : 1.0;
+            b = mid ? 0.5 : 0.0;
+            if (!mid && c + 1 >= sn) c = sn - 2, a = 0.0, b = 1.0;
+          } else {
+            c = (ax == 0 ? X.ax[0].start : (ax == 1 ? X.ax[1].start : X.ax[2].start))[t];
+            const double *w = (ax == 0 ? X.ax[0].w : (ax == 1 ? X.ax[1].w : X.ax[2].w)) + 2 * t;
+            a = w[0];
+            b = w[1];
+          }
+          if (fl & 4u) cc = (ax == 0 ? X.ax[0].coinc : (ax == 1 ? X.ax[1].coinc : X.ax[2].coinc))[t];
+          wi[slot] = a;
+          wf[slot] = b;
+        }
+        // the axis' extent: x over the wave, y and z over lanes 0-3, 4-7
+        int l = v ? (cc >= 0 ? min(c, cc) : c) : 1 << 28, h = v ? max(c + 1, cc) : -1;
+        const int width = wave == 0 ? 64 : 4;
+        for (int d = 1; d < width; d <<= 1) {
+          l = min(l, __shfl_xor(l, d));
+          h = max(h, __shfl_xor(h, d));
+        }
+        if (v) {
+          first[slot] = c - l;
+          same[slot] = cc >= 0 ? cc - l : -1;
+        }
+        if (wave == 0 ? lane == 0 : (lane == 0 || lane == 4)) {
+          lo[ax] = l;
+          ext[ax] = h - l + 1;
+        }
+      }
+    }
+    __syncthreads();
+    fits = fits && ext[0] <= VX && ext[1] <= VY && ext[2] <= VZ;
+    if (fits) {
+      ConstBox &S = cbox(xs[src].src);
+      const void *vf = S.f[F_V];
+      const int ex = ext[0], ey = ext[1], ez = ext[2];
+      // rows of the node block, one a quarter wave: ex <= 36 nodes
+      for (int r = int(threadIdx.x >> 5); r < ey * ez; r += kPtThreads / 32) {
+        const int z = r / ey, y = r - z * ey;
+        for (int x = int(threadIdx.x & 31u); x < ex; x += 32)
+          V[(z * VY + y) * VX + x] = ld<double>(vf, boff(S, lo[0] + x, lo[1] + y, lo[2] + z));
+      }
+      __syncthreads();
+      for (int r = wave; r < ey * ez; r += kPtThreads / 64) {
+        const int z = r / ey, y = r - z * ey;
+        if (vx) {
+          const double *p = V + (z * VY + y) * VX + first[lane];
+          A[(z * VY + y) * TX + lane] = p[0] * wi[lane] + p[1] * wf[lane];
+        }
+      }
+      __syncthreads();
+      if (mine) {
+        const int sy = TX + wave, y0 = first[sy];
+        const double dyi = wi[sy], dyf = wf[sy];
+#pragma unroll
+        for (int q = 0; q < TZ; ++q) {
+          if (q >= nz) break;
+          const int sz = TX + TY + q, z0 = first[sz];
+          double v;
+          if (same[lane] >= 0 && same[sy] >= 0 && same[sz] >= 0) {
+            v = V[(same[sz] * VY + same[sy]) * VX + same[lane]];
+          } else {
+            const double *p = A + (z0 * VY + y0) * TX + lane;
+            v = (p[0] * dyi + p[TX] * dyf) * wi[sz] + (p[VY * TX] * dyi + p[(VY + 1) * TX] * dyf) * wf[sz];
+          }
+          st<double>(T.f[F_U], o[q], u0[q] + v);
+        }
+      }
+    } else if (mine && (mixed || src >= 0)) {
+      for (int q = 0; q < nz; ++q) {
+        const int t[3] = {i, j, k0 + q};
+        for (int x = Bk.nsrc - 1; x >= 0; --x) {
+          ConstXfer &X = xs[x];
+          unsigned fl[3];
+          const unsigned f = axis_flags(X, t, fl);
+          if (!(f & 3)) continue;  // all = true
+          ConstBox &S = cbox(X.src);
+          double v;
+          if (f & 4)
+            v = ld<double>(S.f[F_V], boff(S, X.ax[0].coinc[t[0]], X.ax[1].coinc[t[1]], X.ax[2].coinc[t[2]]));
+          else
+            v = X.affine ? trilinear_nested(S, X, t) : trilinear_corr(S, X, t);
+          const unsigned ot = boff(T, t[0], t[1], t[2]);
+          st<double>(T.f[F_U], ot, ld<double>(T.f[F_U], ot) + v);
+          break;
+        }
+      }
+    }
+    __syncthreads();  // the LDS is reused by the next tile
+  }
 }
 
 // shell point q of a box: the R-thick z slabs first, then y slabs, then x slabs

@@ -460,6 +460,9 @@ inline long long ghost_column_slots(const DevBox &b) {
 inline int robin_edge_sections(const DevBox &B) { return 4 * (B.n[0] + B.n[1] + B.n[2] - 6 * B.R); }
 // target points of one workgroup of a Lagrange transfer (launch_transfer_fields)
 constexpr int kXferTile[3] = {16, 8, 8};
+// fine points of a tile of the prolongation; a PtBlock covers nq planes of
+// tiles from (i0, j0, k0)
+constexpr int kProTile[3] = {64, 4, 4};
 void launch_restrict_u(hipStream_t s, const PtBlock *blocks, int nblocks);
 void launch_restrict_defect(hipStream_t s, const PtBlock *blocks, int nblocks, int order, int eq);
 // generic transfer of field ff of the listed blocks' sources into field

@@ -139,3 +139,42 @@ def test_transfer_tiles(case, order):
                     g, o = h.get_field(ib, oa.F_V), s.field(ib, O.F_V)
                     assert rel_err(g, o) < 1e-12, (frm, to, region, all_, to_zero, ib)
     h.close()
+
+
+@pytest.mark.parametrize("order", [2, 4, 6, 8])
+@pytest.mark.parametrize("eq,n", [(0, 25), (1, 33), (0, 41)])
+def test_paired_operator(eq, n, order):
+    """N(u), dN/du and the mixed-precision defect and update by two slots of
+    a row a thread."""
+    h, s = pair(argv(eq, n, order))
+    seed_state(h, s, 32)
+    for lv in range(s.levels):
+        ng = h.operator(lv)
+        no = max(s.residual(ib) for ib in s.level_boxes(lv))
+        assert abs(ng - no) <= 1e-12 * no, lv
+        for ib in s.level_boxes(lv):
+            R = s.box_info(ib)["R"]
+            inner = (slice(R, -R),) * 3
+            assert rel_err(h.get_field(ib, oa.F_R)[inner], s.field(ib, O.F_R)[inner]) < 1e-12, (lv, ib)
+    # the mixed smoothing of a linear problem (b = 0) is the FP64 one to
+    # single precision: float32 sweeps of the correction, 1e-5 of it
+    p = oa.problem_from_argv(argv(eq, n, order))
+    p.precision = oa.PREC_MIXED
+    m = oa.Hierarchy(p)
+    for ib in range(s.nbox):
+        u = s.field(ib, O.F_U).copy()
+        m.set_field(ib, oa.F_U, u)
+        h.set_field(ib, oa.F_U, u)
+        if eq == 0:
+            for x in (m, h):
+                x.set_field(ib, oa.F_B, np.zeros_like(u))
+    if eq == 0:
+        for lv in range(s.levels):
+            before = [h.get_field(ib, oa.F_U) for ib in s.level_boxes(lv)]
+            m.smooth(lv, 2)
+            h.smooth(lv, 2)
+            for ib, u0 in zip(s.level_boxes(lv), before):
+                a, b = m.get_field(ib, oa.F_U), h.get_field(ib, oa.F_U)
+                assert np.abs(a - b).max() <= 1e-5 * np.abs(b - u0).max(), (lv, ib)
+    m.close()
+    h.close()
