@@ -564,35 +564,77 @@ __device__ __forceinline__ void lap_pair(const void *u, unsigned o, const Nbr<OR
   }
 }
 
+// What a pass by pairs reads of a box descriptor, in scalar registers.
+// load() issues every scalar load at once and waits for them together, with
+// the workgroup's record when the box is known before it (read as they were
+// used, the fields took eight scalar waits in turn).
+struct SweepBox {
+  double *u, *b, *c, *d, *e, *rho;
+  double ix2, iy2, iz2, dulap;
+  unsigned cs, rs, ps;
+  int n0, n1, flip;
+  float inyi;
+  int rlo0, rlo1, rlo2, rhi0, rhi1, rhi2;
+  __device__ __forceinline__ void load(ConstBox &B) {
+    u = B.f[F_U];
+    b = B.f[F_B];
+    c = B.f[F_C];
+    d = B.f[F_D];
+    e = B.f[F_E];
+    rho = B.f[F_RHO];
+    ix2 = B.idx2[0];
+    iy2 = B.idx2[1];
+    iz2 = B.idx2[2];
+    dulap = B.dulap;
+    cs = unsigned(B.cs);
+    rs = unsigned(B.rs);
+    ps = unsigned(B.ps);
+    n0 = B.n[0];
+    n1 = B.n[1];
+    flip = B.flip;
+    inyi = B.inyi;
+    rlo0 = B.rlo[0];
+    rlo1 = B.rlo[1];
+    rlo2 = B.rlo[2];
+    rhi0 = B.rhi[0];
+    rhi1 = B.rhi[1];
+    rhi2 = B.rhi[2];
+  }
+  __device__ __forceinline__ void wait() const {
+    asm volatile("" ::"s"(u), "s"(b), "s"(c), "s"(d), "s"(e), "s"(rho), "s"(ix2), "s"(iy2), "s"(iz2),
+                 "s"(dulap), "s"(cs), "s"(rs), "s"(ps), "s"(n0), "s"(n1), "s"(flip), "s"(inyi),
+                 "s"(rlo0), "s"(rlo1), "s"(rlo2), "s"(rhi0), "s"(rhi1), "s"(rhi2));
+  }
+  // rho of the pair of points (i, j, k), (i + nc, j, k): +0 outside the rho
+  // box, a pair that reaches into it read whole
+  __device__ __forceinline__ void rho_pair(unsigned o, int i, int nc, int j, int k, double r[2]) const {
+    r[0] = r[1] = 0.0;
+    if ((unsigned(j - rlo1) < unsigned(rhi1 - rlo1)) & (unsigned(k - rlo2) < unsigned(rhi2 - rlo2)) &
+        (i + nc >= rlo0) & (i < rhi0))
+      ld_pair(rho, o, r[0], r[1]);
+  }
+};
+
 // N(u) and dN/du of the pair at byte offset o (EQ without first derivatives)
 template <int ORD, int EQ>
-__device__ __forceinline__ void point_op_pair(ConstBox &B, const double *u, unsigned o,
+__device__ __forceinline__ void point_op_pair(const SweepBox &B, unsigned o,
                                               const Nbr<ORD / 2 + 1> &nb, const double u0[2],
                                               double N[2], double dN[2]) {
   double lu[2], b[2], c[2], d[2] = {0.0, 0.0}, e[2] = {0.0, 0.0};
-  ld_pair(B.f[F_B], o, b[0], b[1]);
-  ld_pair(B.f[F_C], o, c[0], c[1]);
+  ld_pair(B.b, o, b[0], b[1]);
+  ld_pair(B.c, o, c[0], c[1]);
   if constexpr (EQ == 1) {
-    ld_pair(B.f[F_D], o, d[0], d[1]);
-    ld_pair(B.f[F_E], o, e[0], e[1]);
+    ld_pair(B.d, o, d[0], d[1]);
+    ld_pair(B.e, o, e[0], e[1]);
   }
-  lap_pair<ORD>(u, o, nb, u0[0], u0[1], B.idx2[0], B.idx2[1], B.idx2[2], lu);
+  lap_pair<ORD>(B.u, o, nb, u0[0], u0[1], B.ix2, B.iy2, B.iz2, lu);
 #pragma unroll
   for (int q = 0; q < 2; ++q)
     nonlinear<EQ>(lu[q], B.dulap, b[q], c[q] + u0[q], d[q], e[q], N[q], dN[q]);
 }
 
-// rho of the pair of points (i, j, k), (i + nc, j, k): +0 outside the rho box
-__device__ __forceinline__ void rho_pair(ConstBox &B, unsigned o, int i, int nc, int j, int k,
-                                         double rho[2]) {
-  rho[0] = rho[1] = 0.0;
-  if ((unsigned(j - B.rlo[1]) < unsigned(B.rhi[1] - B.rlo[1])) &
-      (unsigned(k - B.rlo[2]) < unsigned(B.rhi[2] - B.rlo[2])) & (i + nc >= B.rlo[0]) & (i < B.rhi[0]))
-    ld_pair(B.f[F_RHO], o, rho[0], rho[1]);
-}
-
 template <int ORD, int EQ>
-__device__ __forceinline__ void smooth_pairs(const RowBlock &Bk, ConstBox &B, unsigned per_row,
+__device__ __forceinline__ void smooth_pairs(const RowBlock &Bk, const SweepBox &B, unsigned per_row,
                                              float inv_per_row, int colour) {
   constexpr int R = ORD / 2, NC = R + 1;
   const unsigned lr = fast_div(threadIdx.x, per_row, inv_per_row);
@@ -607,24 +649,24 @@ __device__ __forceinline__ void smooth_pairs(const RowBlock &Bk, ConstBox &B, un
       row /= unsigned(Bk.nseg);
       t += seg * per_row;
     }
-    int j, k;
-    row_jk<R>(B, row, j, k);
+    const unsigned nyi = unsigned(B.n1 - 2 * R);
+    const unsigned kq = fast_div(row, nyi, B.inyi);
+    const int k = R + int(kq), j = R + int(row - kq * nyi);
     const int first = R + int(unsigned(col + NC * 3 * kMaxAxisPoints - j - k - R) % NC);
     const int i = first + int(2 * t) * NC;
-    if (i < B.n[0] - R) {
+    if (i < B.n0 - R) {
       // the second point may be a ghost or padding slot: its loads stay
       // inside the field (rows and planes follow every interior row), and
       // it is neither written nor counted
-      const bool two = i + NC < B.n[0] - R;
-      const unsigned p = unsigned(col) * unsigned(B.cs) + unsigned(k) * unsigned(B.ps) +
-                         unsigned(j) * unsigned(B.rs) + unsigned(first / NC) + 2 * t;
-      const Nbr<NC> nb = box_offs<NC, 8>(B, col, first % NC);
+      const bool two = i + NC < B.n0 - R;
+      const unsigned p = unsigned(col) * B.cs + unsigned(k) * B.ps + unsigned(j) * B.rs +
+                         unsigned(first / NC) + 2 * t;
+      const Nbr<NC> nb = stencil_offs<NC, 8>(col, first % NC, B.cs, B.rs, B.ps);
       const unsigned o = p * 8u;
-      double *u = B.f[F_U];
       double rho[2], u0[2], N[2], dN[2], un[2];
-      rho_pair(B, o, i, NC, j, k, rho);
-      ld_pair(u, o, u0[0], u0[1]);
-      point_op_pair<ORD, EQ>(B, u, o, nb, u0, N, dN);
+      B.rho_pair(o, i, NC, j, k, rho);
+      ld_pair(B.u, o, u0[0], u0[1]);
+      point_op_pair<ORD, EQ>(B, o, nb, u0, N, dN);
 #pragma unroll
       for (int q = 0; q < 2; ++q) {
         const double res = N[q] - rho[q];
@@ -635,40 +677,46 @@ __device__ __forceinline__ void smooth_pairs(const RowBlock &Bk, ConstBox &B, un
         }
       }
       if (two)
-        st_pair(u, o, un[0], un[1]);
+        st_pair(B.u, o, un[0], un[1]);
       else
-        st<double>(u, o, un[0]);
+        st<double>(B.u, o, un[0]);
     }
   }
   wave_norm(Bk.norm, rmax, seen);
 }
 
-template <int ORD, int EQ>
-__device__ __forceinline__ void smooth_block(const RowBlock &Bk, ConstBox &B, unsigned per_row,
-                                             float inv_per_row, int colour) {
-  if constexpr (sweep_points(EQ) == 2)
-    smooth_pairs<ORD, EQ>(Bk, B, per_row, inv_per_row, colour);
-  else
-    smooth_rows<ORD, EQ>(Bk, B, per_row, inv_per_row, colour);
-}
-
 // box1: the one box of every listed block, when the launch covers a single
 // box (else null); its descriptor is then fetched without waiting for the
-// block's.  Either way the descriptor's cache lines are fetched in one batch
-// first: the kernel branches on several of its fields, and loads issued
-// branch by branch would each wait for the one before.
+// block's.
+// Four waves per SIMD leave a wave the registers to issue its loads (17 at
+// 4th, 25 at 6th, 29 at 8th order) before it waits for the first; compiled
+// for more waves it issued 11 to 14 and waited.  With the scalar loads
+// together (SweepBox): N=161 smoother 94.2 -> 90.3 ms per two V-cycles, 16 x
+// N=65 23.8 -> 23.1, N=129 8th order 21.3 -> 20.4, one 33^3 solve 6.40 ->
+// 6.28.
 template <int ORD, int EQ>
-__global__ __launch_bounds__(kMaxRowThreads) void k_smooth(const RowBlock *__restrict__ blocks,
+__global__ __launch_bounds__(kMaxRowThreads) __attribute__((amdgpu_waves_per_eu(4, 4)))
+void k_smooth(const RowBlock *__restrict__ blocks,
                                                         unsigned per_row, float inv_per_row,
                                                         int colour, const DevBox *box1) {
-  if (box1) {
-    const RowBlock Bk = blocks[xcd_block()];
-    fetch_box(box1);
-    smooth_block<ORD, EQ>(Bk, cbox(box1), per_row, inv_per_row, colour);
+  if constexpr (sweep_points(EQ) == 2) {
+    RowBlock Bk;
+    SweepBox B;
+    if (box1) {
+      B.load(cbox(box1));
+      Bk = blocks[xcd_block()];
+      B.wait();
+    } else {
+      Bk = blocks[xcd_block()];
+      B.load(cbox(Bk.box));
+      B.wait();
+    }
+    smooth_pairs<ORD, EQ>(Bk, B, per_row, inv_per_row, colour);
   } else {
     const RowBlock Bk = blocks[xcd_block()];
-    fetch_box(Bk.box);
-    smooth_block<ORD, EQ>(Bk, cbox(Bk.box), per_row, inv_per_row, colour);
+    const DevBox *box = box1 ? box1 : Bk.box;
+    fetch_box(box);
+    smooth_rows<ORD, EQ>(Bk, cbox(box), per_row, inv_per_row, colour);
   }
 }
 
@@ -827,6 +875,8 @@ __global__ __launch_bounds__(kRowThreads) void k_residual(const RowBlock *__rest
   if constexpr (sweep_points(EQ) == 2) {
     // two slots a thread, as the colour passes (one: N=161 6th order 234 us a
     // launch, 16 x N=65 4th order 67; two: 188 and 53)
+    SweepBox P;
+    P.load(B);
     double *out = mode == RES_DEFECT ? B.f[F_W] : B.f[F_R];
     for_rows(Bk, per_row, inv_per_row, [&](unsigned rpb, unsigned lr0) {
       unsigned p;
@@ -835,11 +885,10 @@ __global__ __launch_bounds__(kRowThreads) void k_residual(const RowBlock *__rest
       if (!row_pair<R>(Bk, B, per_row, inv_per_row, rpb, lr0, p, c, s, i, j, k, ok)) return;
       const Nbr<R + 1> nb = box_offs<R + 1, 8>(B, c, s);
       const unsigned o = p * 8u;
-      const double *u = B.f[F_U];
       double rho[2] = {0.0, 0.0}, u0[2], N[2], dN[2], v[2];
-      if (mode == RES_DEFECT) rho_pair(B, o, i, R + 1, j, k, rho);
-      ld_pair(u, o, u0[0], u0[1]);
-      point_op_pair<ORD, EQ>(B, u, o, nb, u0, N, dN);
+      if (mode == RES_DEFECT) P.rho_pair(o, i, R + 1, j, k, rho);
+      ld_pair(P.u, o, u0[0], u0[1]);
+      point_op_pair<ORD, EQ>(P, o, nb, u0, N, dN);
 #pragma unroll
       for (int q = 0; q < 2; ++q) {
         v[q] = mode == RES_DEFECT ? rho[q] - N[q] : (mode == RES_DERIVATIVE ? dN[q] : N[q]);
@@ -889,6 +938,8 @@ __global__ __launch_bounds__(kRowThreads) void k_defect32(const RowBlock *__rest
   const RowBlock Bk = blocks[xcd_block()];
   ConstBox &B = cbox(Bk.box);
   const double seen = norm_seen(Bk.norm);
+  SweepBox P;
+  P.load(B);
   double rmax = 0.0;
   for_rows(Bk, per_row, inv_per_row, [&](unsigned rpb, unsigned lr0) {
     unsigned p;
@@ -897,11 +948,10 @@ __global__ __launch_bounds__(kRowThreads) void k_defect32(const RowBlock *__rest
     if (!row_pair<R>(Bk, B, per_row, inv_per_row, rpb, lr0, p, c, s, i, j, k, ok)) return;
     const Nbr<NC> nb = box_offs<NC, 8>(B, c, s);
     const unsigned o = p * 8u;
-    const double *u = B.f[F_U];
     double rho[2], u0[2], N[2], dN[2];
-    rho_pair(B, o, i, NC, j, k, rho);
-    ld_pair(u, o, u0[0], u0[1]);
-    point_op_pair<ORD, EQ>(B, u, o, nb, u0, N, dN);
+    P.rho_pair(o, i, NC, j, k, rho);
+    ld_pair(P.u, o, u0[0], u0[1]);
+    point_op_pair<ORD, EQ>(P, o, nb, u0, N, dN);
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
       if (!ok[q]) continue;
