@@ -1136,23 +1136,25 @@ struct Builder {
 
   void coarse(const std::vector<Hier *> &M) {
     std::map<int, std::vector<CoarseItem>> groups;  // eq -> items
-    std::map<int, std::pair<int, int>> sizes;
+    std::map<int, std::array<int, 3>> sizes;
     for (Hier *H : M) {
       const int b0 = H->geo.level_first[0];
       const DevBox &B = H->hbox[size_t(b0)];
       groups[H->prob.eq].push_back(CoarseItem{H->dbox + b0, H->slot(Hier::slot_pre(0)), H->iters,
                                               H->coarse_omega});
       auto &sz = sizes[H->prob.eq];
-      sz.first = std::max<int>(sz.first, int(B.size));
-      sz.second = std::max<int>(sz.second, int(coarse_colour_slots(B.n)));
+      sz[0] = std::max<int>(sz[0], int(B.size));
+      sz[1] = std::max<int>(sz[1], int(coarse_colour_slots(B.n)));
+      sz[2] = std::max<int>(sz[2], int(coarse_shell_points(B.n)));
     }
     for (auto &g : groups) {
       Launch L{Launch::COARSE};
       L.eq = g.first;
       L.off = S.add(g.second);
       L.n = int(g.second.size());
-      L.max_pts = sizes[g.first].first;
-      L.max_int = sizes[g.first].second;
+      L.max_pts = sizes[g.first][0];
+      L.max_int = sizes[g.first][1];
+      L.max_row = sizes[g.first][2];
       S.launches.push_back(L);
     }
   }
@@ -1309,7 +1311,7 @@ int issue(const Schedule &S, hipStream_t s, Timing *t, std::string &err) {
         break;
       case Launch::COARSE:
         if (!launch_coarse_solve(s, reinterpret_cast<const CoarseItem *>(items), L.n, L.max_pts,
-                                 L.max_int, L.eq, 2 * DBL_EPSILON, 100000))
+                                 L.max_int, L.max_row, L.eq, 2 * DBL_EPSILON, 100000))
           return err = "coarsest box exceeds the LDS of one workgroup", OLL_EINVAL;
         break;
       case Launch::CORR_V:

@@ -102,7 +102,7 @@ struct Launch {
   size_t off = 0;     // items in the schedule blob
   int n = 0;          // items
   long long total = 0;
-  int max_row = 0;    // row kernels: threads per row
+  int max_row = 0;    // row kernels: threads per row; COARSE: largest shell
   int threads = kRowThreads;  // colour passes: threads per workgroup
   int max_pts = 0, max_int = 0;  // COARSE: largest box, colour slot list; ROBIN: edge cross-sections
   int pair = 0, parity = 0;  // SMOOTH_FUSED: two passes or one; 0 reads u, 1 reads r

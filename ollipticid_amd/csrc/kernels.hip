@@ -333,18 +333,43 @@ __device__ __forceinline__ double dpp_f64(double v) {
   return __longlong_as_double((long long)(((unsigned long long)(unsigned)h2 << 32) | (unsigned)l2));
 }
 
-// max over the 64 lanes of a wave (all lanes active); uniform result
-__device__ __forceinline__ double wave_max_dpp(double v) {
-  v = fmax(v, dpp_f64<0xB1, 0xF>(v));   // quad_perm [1,0,3,2]
-  v = fmax(v, dpp_f64<0x4E, 0xF>(v));   // quad_perm [2,3,0,1]
-  v = fmax(v, dpp_f64<0x141, 0xF>(v));  // row_half_mirror
-  v = fmax(v, dpp_f64<0x140, 0xF>(v));  // row_mirror
-  v = fmax(v, dpp_f64<0x142, 0xA>(v));  // row_bcast15
-  v = fmax(v, dpp_f64<0x143, 0xC>(v));  // row_bcast31: lane 63 holds the max
-  const long long b = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_readlane(int(b), 63);
-  const int hi = __builtin_amdgcn_readlane(int(b >> 32), 63);
-  return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
+// Max of doubles none of which is negative or NaN, which order as their bits
+// do: of the upper words first, then of the lower words beside the largest
+// upper one: 14 instructions over a wave where the maxima of doubles take
+// 36.  All lanes of the wave must be active.
+template <int CTRL, int ROW_MASK>
+__device__ __forceinline__ unsigned dpp_max_u32(unsigned v) {
+  const unsigned w = unsigned(__builtin_amdgcn_update_dpp(0, int(v), CTRL, ROW_MASK, 0xF, false));
+  return v > w ? v : w;
+}
+// over N = 8 or 16 lanes of a row that hold the same in every row
+template <int N>
+__device__ __forceinline__ unsigned row_max_u32(unsigned v) {
+  v = dpp_max_u32<0xB1, 0xF>(v);
+  v = dpp_max_u32<0x4E, 0xF>(v);
+  v = dpp_max_u32<0x141, 0xF>(v);
+  if constexpr (N == 16) v = dpp_max_u32<0x140, 0xF>(v);
+  return v;
+}
+__device__ __forceinline__ unsigned wave_max_u32(unsigned v) {
+  v = row_max_u32<16>(v);
+  v = dpp_max_u32<0x142, 0xA>(v);
+  v = dpp_max_u32<0x143, 0xC>(v);
+  return unsigned(__builtin_amdgcn_readlane(int(v), 63));
+}
+__device__ __forceinline__ double wave_max_pos(double v) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  const unsigned hi = wave_max_u32(unsigned(b >> 32));
+  const unsigned lo = wave_max_u32(unsigned(b >> 32) == hi ? unsigned(b) : 0u);
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+template <int N>
+__device__ __forceinline__ double row_max_pos(double v) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  const unsigned hi = row_max_u32<N>(unsigned(b >> 32));
+  const unsigned lo = row_max_u32<N>(unsigned(b >> 32) == hi ? unsigned(b) : 0u);
+  const int h = __builtin_amdgcn_readfirstlane(int(hi)), l = __builtin_amdgcn_readfirstlane(int(lo));
+  return __longlong_as_double((long long)(((unsigned long long)unsigned(h) << 32) | unsigned(l)));
 }
 
 // what the block's norm slot holds as the block starts (thread 0; 0 without
@@ -364,7 +389,7 @@ __device__ __forceinline__ double norm_seen(const unsigned long long *slot) {
 // slot already held `seen` >= the maximum
 __device__ __forceinline__ void wave_norm(unsigned long long *slot, double v, double seen) {
   __shared__ double sh[kMaxRowThreads / 64];
-  const double m = wave_max_dpp(v);
+  const double m = wave_max_pos(v);
   if (blockDim.x == 64) {
     if (threadIdx.x == 0 && slot && m > seen) norm_update(slot, m);
     return;
@@ -2603,54 +2628,10 @@ __device__ __forceinline__ int coarse_p(const CoarseGeo &G, int i, int j, int k)
   return c * G.cs + k * G.ps + j * G.rs + int((unsigned(i) * G.ncm) >> 16);
 }
 
-// Robin update at shell point (i, j, k) of the LDS field; mask has bit a
-// for each axis whose index is 0 or n-1 (dx2 one-sided derivative,
-// diff_2nd.cc:237-335).  The coarsest level is 2nd order, so its layout has
-// two colours: point (i, j, k) is slot i / 2 of row (j, k) in block
-// (i + j + k) & 1, and a step along an axis moves to the other block.
-__device__ __forceinline__ void coarse_robin(const CoarseGeo &G, double *su, const double *srho,
-                                             int i, int j, int k, int mask) {
-  const int c = (i + j + k) & 1;
-  const int p = c * G.cs + k * G.ps + j * G.rs + (i >> 1);
-  const int flip = (1 - 2 * c) * G.cs;
-  const int ijk[3] = {i, j, k};
-  double X[3];
-#pragma unroll
-  for (int a = 0; a < 3; ++a) X[a] = G.lo[a] + (double)ijk[a] * G.d[a];
-  const double r2 = X[0] * X[0] + X[1] * X[1] + X[2] * X[2];
-  double sF = 0.0, sdF = 0.0;
-#pragma unroll
-  for (int a = 0; a < 3; ++a) {
-    if (!(mask & (1 << a))) continue;
-    const bool lo = ijk[a] == 0;
-    const int dir = lo ? 1 : -1;
-    // offsets of the points 1 and 2 steps inwards along axis a
-    int o1, o2;
-    if (a == 0) {
-      o1 = flip + ((i + dir) >> 1) - (i >> 1);
-      o2 = dir;
-    } else {
-      const int st = a == 1 ? G.rs : G.ps;
-      o1 = flip + dir * st;
-      o2 = 2 * dir * st;
-    }
-    const double id = G.idx[a];
-    double cf, dv;
-    if (lo) {
-      cf = -3.0 * 0.5 * id;
-      dv = (-3.0 * su[p] + 4.0 * su[p + o1] - su[p + o2]) * 0.5 * id;
-    } else {
-      cf = 3.0 * 0.5 * id;
-      dv = (3.0 * su[p] - 4.0 * su[p + o1] + su[p + o2]) * 0.5 * id;
-    }
-    sF += dv / X[a];
-    sdF += cf / X[a];
-  }
-  const double op = r2 * G.ipn * sF + su[p];
-  const double Fv = op - srho[p];
-  const double dF = r2 * G.ipn * sdF + 1.0;
-  su[p] = su[p] - Fv / dF;
-}
+// The Robin updates of the shell (one-sided derivative dx2, diff_2nd.cc:237-335).
+// The coarsest level is 2nd order, so its layout has two colours: point
+// (i, j, k) is slot i / 2 of row (j, k) in block (i + j + k) & 1, and a step
+// along an axis moves to the other block.
 
 // face point t of the coarsest box (x faces, then y, then z, low side
 // first): (i, j, k) and its side, 2 axis + high
@@ -2680,41 +2661,105 @@ __device__ __forceinline__ int coarse_face(const CoarseGeo &G, int t, float ini,
   return 4 + hi;
 }
 
-// a / b from y = 1 / b: the quotient corrected by its exact remainder
-// (Markstein 1990)
+// a / b from y = 1 / b (rounded): the quotient corrected twice by its exact
+// remainder.  a y may be two units off, one correction brings it within one,
+// and from there the second rounds as the division does (Markstein 1990);
+// zeros, infinities and NaN as the division has them
 __device__ __forceinline__ double div_by(double a, double b, double y) {
-  const double q = a * y;
-  return fma(fma(-q, b, a), y, q);
+  double q = a * y;
+  q = fma(fma(-q, b, a), y, q);
+  return __builtin_amdgcn_div_fixup(fma(fma(-q, b, a), y, q), b, a);
 }
-// a / b by two Newton steps on the hardware reciprocal and the same
-// correction; zeros, infinities and NaN as the division has them.  The
-// coarsest solve's quotients are far from the exponents' limits, so the
-// scaling steps of the general division (2 of its 11) are left out.
+// a / b by two Newton steps on the hardware reciprocal and one correction;
+// zeros, infinities and NaN as the division has them.  The coarsest solve's
+// quotients are far from the exponents' limits, so the scaling steps of the
+// general division (2 of its 11) are left out; the rest are its own, to the
+// bit.
 __device__ __forceinline__ double div_newton(double a, double b) {
   double y = __builtin_amdgcn_rcp(b);
   y = fma(fma(-b, y, 1.0), y, y);
   y = fma(fma(-b, y, 1.0), y, y);
-  return __builtin_amdgcn_div_fixup(div_by(a, b, y), b, a);
+  const double q = a * y;
+  return __builtin_amdgcn_div_fixup(fma(fma(-q, b, a), y, q), b, a);
+}
+
+// edge t of the coarsest box (XY, XZ, YZ edges) or, with CORNER, corner t:
+// (i, j, k) and its sides in the order of their axes
+template <bool CORNER>
+__device__ __forceinline__ void coarse_edge(const CoarseGeo &G, int t, int ijk[3], int sd[3]) {
+  const int ni = G.n[0] - 2, nj = G.n[1] - 2, nk = G.n[2] - 2;
+  if (CORNER) {
+    sd[0] = (t >> 1) & 1;
+    sd[1] = 2 + (t >> 2);
+    sd[2] = 4 + (t & 1);
+  } else if (t < 4 * nk) {
+    const int e = (t >= nk) + (t >= 2 * nk) + (t >= 3 * nk);
+    sd[0] = e >> 1;
+    sd[1] = 2 + (e & 1);
+    ijk[2] = 1 + t - e * nk;
+  } else if ((t -= 4 * nk) < 4 * nj) {
+    const int e = (t >= nj) + (t >= 2 * nj) + (t >= 3 * nj);
+    sd[0] = e >> 1;
+    sd[1] = 4 + (e & 1);
+    ijk[1] = 1 + t - e * nj;
+  } else {
+    t -= 4 * nj;
+    const int e = (t >= ni) + (t >= 2 * ni) + (t >= 3 * ni);
+    sd[0] = 2 + (e & 1);
+    sd[1] = 4 + (e >> 1);
+    ijk[0] = 1 + t - e * ni;
+  }
+#pragma unroll
+  for (int a = 0; a < 3; ++a)
+#pragma unroll
+    for (int m = 0; m < (CORNER ? 3 : 2); ++m)
+      if ((sd[m] >> 1) == a) ijk[a] = (sd[m] & 1) ? G.n[a] - 1 : 0;
+}
+
+// r^2 / n at (i, j, k)
+__device__ __forceinline__ double coarse_r2n(const CoarseGeo &G, int i, int j, int k) {
+  const double X0 = G.lo[0] + (double)i * G.d[0], X1 = G.lo[1] + (double)j * G.d[1],
+               X2 = G.lo[2] + (double)k * G.d[2];
+  return (X0 * X0 + X1 * X1 + X2 * X2) * G.ipn;
+}
+
+// index of the point one step inwards from (i, j, k) at side sd
+__device__ __forceinline__ int coarse_in(const CoarseGeo &G, int i, int j, int k, int sd) {
+  const int dir = (sd & 1) ? -1 : 1, ax = sd >> 1;
+  return coarse_p(G, i + (ax == 0 ? dir : 0), j + (ax == 1 ? dir : 0), k + (ax == 2 ? dir : 0));
+}
+
+// One side's derivative at the point at index p (p1: one step inwards) over
+// X.  Two steps inwards lie in p's own colour block: one slot, two rows or
+// two planes on.
+__device__ __forceinline__ double coarse_side(const CoarseGeo &G, const double (*side)[4],
+                                              const double *su, double u0, int p, int p1, int sd) {
+  const int st = sd < 2 ? 1 : 2 * (sd < 4 ? G.rs : G.ps);
+  const int p2 = p + ((sd & 1) ? -st : st);
+  const double dv = (-3.0 * u0 + 4.0 * su[p1] - su[p2]) * 0.5 * side[sd][2];
+  const double q = div_by(dv, side[sd][0], side[sd][1]);
+  __builtin_amdgcn_sched_barrier(0);  // one side at a time: fewer registers
+  return q;
 }
 
 // One workgroup and its CU carry a box's whole loop, so the kernel is bound
 // by the double-precision instructions it issues per sweep, not by memory.
-// - An interior point reads the shell's faces only, never its edges and
-//   corners, and an edge or corner point's update solves its linear Robin
-//   equation whatever the point held before: edges and corners are updated
-//   once, after the last sweep, from the faces that sweep read.
 // - Each thread keeps what does not change of its face points: the indices,
-//   r^2 / n, dF and 1 / dF (the divisions become a product and two fma).
-// 17^3 4.9 -> 2.6 us a sweep, 21^3 with the scalar field 8.5 -> 6.9 us.
-// FACES: face points a thread keeps; those beyond (flat boxes) are decoded
-// and updated each sweep.
+//   r^2 / n, dF and 1 / dF (a division becomes a product, four fma and the
+//   fix-up, and rounds the same).
+// - An interior point reads the shell's faces only, never its edges and
+//   corners.  The edges are updated beside the first colour pass and the
+//   corners beside the second, without barriers of their own, by the last
+//   waves, which have an interior point less.  An edge's constants take the
+//   place of the last waves' missing face point, the corners' lie in LDS.
+// FACES: face points a thread keeps.  The threads hold all face and edge
+// points (FACES * NT): loops for points beyond them, though never entered,
+// took registers and scalar registers enough to make the kernel spill.
 // OWN: interior points per colour per thread (colour c's points are
-// numbered row by row, ceil(ni / 2) slots per interior row).  With at most
-// 2048 points per colour over the workgroup (OWN * NT) the coefficients of
-// a thread's points stay in registers for the whole loop; beyond that they
-// would not fit the register file (the kernel spilled), so each point's
-// coefficients are loaded from the (cache-resident) fields as the point is
-// updated.
+// numbered row by row, ceil(ni / 2) slots per interior row).  The
+// coefficients of a thread's points stay in registers for the whole loop
+// where they fit the register file; otherwise each point's are loaded from
+// the (cache-resident) fields as the point is updated.
 template <int EQ, int OWN, int NT, int FACES>
 __global__ __launch_bounds__(NT) void k_coarse_solve(const CoarseItem *__restrict__ items,
                                                                  double eps, int max_iter) {
@@ -2754,8 +2799,10 @@ __global__ __launch_bounds__(NT) void k_coarse_solve(const CoarseItem *__restric
   const int ni = n0 - 2, nj = n1 - 2, nk = n2 - 2;
   const int per_row = (ni + 1) / 2;
   const int slots = nj * nk * per_row;
-  constexpr bool kCached = OWN * NT <= 2048;
+  constexpr bool kLong = EQ == 1 || EQ == kEqPuncturesEm;  // more coefficients a point
+  constexpr bool kCached = OWN * NT <= 2048 || EQ == 0;
   constexpr int NCACHE = kCached ? 2 * OWN : 1;
+  constexpr bool kKeepAddr = OWN * NT <= 2048 && !kLong;
   int own_p[2 * OWN];
   double own_b[NCACHE], own_cc[NCACHE], own_d[NCACHE], own_e[NCACHE];
   // the coefficients of owned point q (colour col, slot m)
@@ -2787,15 +2834,17 @@ __global__ __launch_bounds__(NT) void k_coarse_solve(const CoarseItem *__restric
     }
   // shell points: faces (x, y, z pairs), edges (XY, XZ, YZ), corners
   const int nface = 2 * (nj * nk + ni * nk + ni * nj), nedge = 4 * (ni + nj + nk);
-  const float ini = 1.0f / float(ni), inj = 1.0f / float(nj), ink = 1.0f / float(nk);
-  // per side (2 axis + high): coordinate X, 1 / X and 1 / d signed inwards
-  __shared__ double side[6][3];
+  const float ini = 1.0f / float(ni), inj = 1.0f / float(nj);
+  // per side (2 axis + high): coordinate X, 1 / X, 1 / d signed inwards and
+  // the side's term of dF
+  __shared__ double side[6][4];
   if (threadIdx.x < 6) {
     const int ax = threadIdx.x >> 1, hi = threadIdx.x & 1;
     const double X = B.lo[ax] + double(hi ? B.n[ax] - 1 : 0) * B.d[ax];
     side[threadIdx.x][0] = X;
     side[threadIdx.x][1] = 1.0 / X;
     side[threadIdx.x][2] = hi ? -B.idx[ax] : B.idx[ax];
+    side[threadIdx.x][3] = -3.0 * 0.5 * side[threadIdx.x][2] / X;
   }
   __syncthreads();
   // owned face points: index | side << 16 (-1: none), indices of the two
@@ -2813,18 +2862,42 @@ __global__ __launch_bounds__(NT) void k_coarse_solve(const CoarseItem *__restric
     int i, j, k;
     const int sd = coarse_face(G, t, ini, inj, i, j, k);
     const int dir = (sd & 1) ? -1 : 1, ax = sd >> 1;
-    const double X0 = G.lo[0] + (double)i * G.d[0], X1 = G.lo[1] + (double)j * G.d[1],
-                 X2 = G.lo[2] + (double)k * G.d[2];
-    const double r2 = X0 * X0 + X1 * X1 + X2 * X2;
-    const double cf = -3.0 * 0.5 * side[sd][2];
     face_p[m] = coarse_p(G, i, j, k) | (sd << 16);
-    const int p1 = coarse_p(G, i + (ax == 0 ? dir : 0), j + (ax == 1 ? dir : 0), k + (ax == 2 ? dir : 0));
     const int p2 = coarse_p(G, i + (ax == 0 ? 2 * dir : 0), j + (ax == 1 ? 2 * dir : 0),
                             k + (ax == 2 ? 2 * dir : 0));
-    face_in[m] = unsigned(p1) | (unsigned(p2) << 16);
-    face_a[m] = r2 * G.ipn;
-    face_df[m] = r2 * G.ipn * (cf / side[sd][0]) + 1.0;
+    face_in[m] = unsigned(coarse_in(G, i, j, k, sd)) | (unsigned(p2) << 16);
+    face_a[m] = coarse_r2n(G, i, j, k);
+    face_df[m] = face_a[m] * side[sd][3] + 1.0;
     face_y[m] = 1.0 / face_df[m];
+  }
+  // edge points: thread NT - 1 - t keeps edge t as its last face point (the
+  // host sees to it that no thread that takes an edge has one there); corner
+  // points: one of eight threads each
+  const int et = NT - 1 - int(threadIdx.x);
+  const bool edge = et < nedge;
+  if (edge) {
+    int ijk[3], sd[3];
+    coarse_edge<false>(G, et, ijk, sd);
+    face_p[FACES - 1] = coarse_p(G, ijk[0], ijk[1], ijk[2]) | (sd[0] << 16) | (sd[1] << 20);
+    face_in[FACES - 1] = unsigned(coarse_in(G, ijk[0], ijk[1], ijk[2], sd[0])) |
+                         unsigned(coarse_in(G, ijk[0], ijk[1], ijk[2], sd[1])) << 16;
+    face_a[FACES - 1] = coarse_r2n(G, ijk[0], ijk[1], ijk[2]);
+    face_df[FACES - 1] = face_a[FACES - 1] * (side[sd[0]][3] + side[sd[1]][3]) + 1.0;
+    face_y[FACES - 1] = 1.0 / face_df[FACES - 1];
+  }
+  __shared__ double corner[8][3];  // r^2 / n, dF, 1 / dF
+  __shared__ int corner_p[8][7];   // index, one step inwards per axis, sides
+  if (et < 8) {
+    int ijk[3], sd[3];
+    coarse_edge<true>(G, et, ijk, sd);
+    corner_p[et][0] = coarse_p(G, ijk[0], ijk[1], ijk[2]);
+    for (int a = 0; a < 3; ++a) {
+      corner_p[et][1 + a] = coarse_in(G, ijk[0], ijk[1], ijk[2], sd[a]);
+      corner_p[et][4 + a] = sd[a];
+    }
+    corner[et][0] = coarse_r2n(G, ijk[0], ijk[1], ijk[2]);
+    corner[et][1] = corner[et][0] * (side[sd[0]][3] + side[sd[1]][3] + side[sd[2]][3]) + 1.0;
+    corner[et][2] = 1.0 / corner[et][1];
   }
   double prev = 1.0, cur = 1.0;
   int it = 0;
@@ -2832,17 +2905,12 @@ __global__ __launch_bounds__(NT) void k_coarse_solve(const CoarseItem *__restric
     prev = cur;
 #pragma unroll
     for (int m = 0; m < FACES; ++m) {
-      if (face_p[m] < 0) continue;
+      if (face_p[m] < 0 || (m == FACES - 1 && edge)) continue;
       const int p = face_p[m] & 0xffff, sd = face_p[m] >> 16;
       const double u0 = su[p];
       const double dv = (-3.0 * u0 + 4.0 * su[face_in[m] & 0xffffu] - su[face_in[m] >> 16]) * 0.5 * side[sd][2];
       const double op = face_a[m] * div_by(dv, side[sd][0], side[sd][1]) + u0;
       su[p] = u0 - div_by(op - srho[p], face_df[m], face_y[m]);
-    }
-    for (int t = threadIdx.x + FACES * NT; t < nface; t += NT) {
-      int i, j, k;
-      const int sd = coarse_face(G, t, ini, inj, i, j, k);
-      coarse_robin(G, su, srho, i, j, k, 1 << (sd >> 1));
     }
     __syncthreads();
     double mx = 0.0;
@@ -2862,25 +2930,33 @@ __global__ __launch_bounds__(NT) void k_coarse_solve(const CoarseItem *__restric
         } else {
           coeffs(q, qb, qc, qd, qe);
         }
-        const int p = own_p[q] & 0x3fffffff;
-        const Nbr<2> nb = stencil_offs<2, 1>(col, own_p[q] >> 30, unsigned(G.cs), unsigned(G.rs),
-                                             unsigned(G.ps));
-        const double lu = lap<2>(su, p, nb, G.idx2[0], G.idx2[1], G.idx2[2]);
+        // the neighbours' addresses stay in registers over the loop where
+        // there are enough (formed each sweep, 17^3 takes 3.4 us a sweep
+        // instead of 3.1; spilled, 21^3 with the scalar field takes 8.6
+        // instead of 7.2)
+        int po = own_p[q];
+        if constexpr (!kKeepAddr) asm volatile("" : "+v"(po));
+        const int p = po & 0x3fffffff;
+        const Nbr<2> nb = stencil_offs<2, 1>(col, po >> 30, unsigned(G.cs), unsigned(G.rs), unsigned(G.ps));
+        const double u0 = su[p], xp = su[p + int(nb.xp[0])], xm = su[p + int(nb.xm[0])],
+                     yp = su[p + int(nb.yp[0])], ym = su[p + int(nb.ym[0])],
+                     zp = su[p + int(nb.zp[0])], zm = su[p + int(nb.zm[0])], rho = srho[p];
+        const double lu = star_sum<2, double>(fma(-2.0, u0, xp + xm), fma(-2.0, u0, yp + ym),
+                                              fma(-2.0, u0, zp + zm), G.idx2[0], G.idx2[1], G.idx2[2]);
         double N, dN;
         if constexpr (EQ == kEqPuncturesEm) {
           const unsigned o = unsigned(p) * 8u;
-          const double g[3] = {(su[p + int(nb.xp[0])] - su[p + int(nb.xm[0])]) * 0.5 * G.idx[0],
-                               (su[p + int(nb.yp[0])] - su[p + int(nb.ym[0])]) * 0.5 * G.idx[1],
-                               (su[p + int(nb.zp[0])] - su[p + int(nb.zm[0])]) * 0.5 * G.idx[2]};
+          const double g[3] = {(xp - xm) * 0.5 * G.idx[0], (yp - ym) * 0.5 * G.idx[1],
+                               (zp - zm) * 0.5 * G.idx[2]};
           const double ge[3] = {ld<double>(B.f[F_X0], o), ld<double>(B.f[F_X1], o), ld<double>(B.f[F_X2], o)};
           const double gf[3] = {ld<double>(B.f[F_X3], o), ld<double>(B.f[F_X4], o), ld<double>(B.f[F_X5], o)};
           const double du[3] = {0.0, 0.0, 0.0};  // order 2: centred derivatives
-          em_nonlinear(lu, G.dulap, su[p], g, du, qb, qd, ge, gf, N, dN);
+          em_nonlinear(lu, G.dulap, u0, g, du, qb, qd, ge, gf, N, dN);
         } else {
-          nonlinear<EQ, true>(lu, G.dulap, qb, qc + su[p], qd, qe, N, dN);
+          nonlinear<EQ, true>(lu, G.dulap, qb, qc + u0, qd, qe, N, dN);
         }
-        const double res = N - srho[p];
-        const double un = su[p] - omega * div_newton(res, dN);
+        const double res = N - rho;
+        const double un = u0 - omega * div_newton(res, dN);
         su[p] = un;
         mx = fmax(mx, fabs(res));
         if (!(un == un)) mx = __longlong_as_double(0x7ff0000000000000LL);
@@ -2888,36 +2964,37 @@ __global__ __launch_bounds__(NT) void k_coarse_solve(const CoarseItem *__restric
         // otherwise be interleaved past the register budget)
         __builtin_amdgcn_sched_barrier(0);
       }
-      if (col == 0) __syncthreads();
+      if (col == 0) {
+        if (edge) {
+          constexpr int m = FACES - 1;
+          int fp = face_p[m];
+          asm volatile("" : "+v"(fp));
+          const int p = fp & 0xffff;
+          const double u0 = su[p];
+          const double sF =
+              coarse_side(G, side, su, u0, p, int(face_in[m] & 0xffffu), (fp >> 16) & 15) +
+              coarse_side(G, side, su, u0, p, int(face_in[m] >> 16), fp >> 20);
+          su[p] = u0 - div_by(face_a[m] * sF + u0 - srho[p], face_df[m], face_y[m]);
+        }
+        __syncthreads();
+      } else if (et < 8) {
+        int tc = NT - 1 - int(threadIdx.x);
+        asm volatile("" : "+v"(tc));
+        const int *c = corner_p[tc];
+        const int p = c[0];
+        const double u0 = su[p];
+        double sF = coarse_side(G, side, su, u0, p, c[1], c[4]);
+        sF += coarse_side(G, side, su, u0, p, c[2], c[5]);
+        sF += coarse_side(G, side, su, u0, p, c[3], c[6]);
+        su[p] = u0 - div_by(corner[tc][0] * sF + u0 - srho[p], corner[tc][1], corner[tc][2]);
+      }
     }
-    const double wm = wave_max_dpp(mx);
+    const double wm = wave_max_pos(mx);
     if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = wm;
     __syncthreads();
-    cur = sh[0];
-#pragma unroll
-    for (int w = 1; w < NT / 64; ++w) cur = fmax(cur, sh[w]);
+    cur = row_max_pos<NT / 64>(sh[threadIdx.x & (NT / 64 - 1)]);
     ++it;
   } while (cur > eps && prev != cur && it < max_iter && !isinf(cur));
-  for (int t = threadIdx.x; t < nedge; t += NT) {
-    int r = t, i, j, k, mask;
-    if (r < 4 * nk) {
-      const int e = int(fast_div(unsigned(r), unsigned(nk), ink));
-      i = (e >> 1) ? n0 - 1 : 0; j = (e & 1) ? n1 - 1 : 0; k = 1 + r - e * nk; mask = 3;
-    } else if ((r -= 4 * nk) < 4 * nj) {
-      const int e = int(fast_div(unsigned(r), unsigned(nj), inj));
-      i = (e >> 1) ? n0 - 1 : 0; k = (e & 1) ? n2 - 1 : 0; j = 1 + r - e * nj; mask = 5;
-    } else {
-      r -= 4 * nj;
-      const int e = int(fast_div(unsigned(r), unsigned(ni), ini));
-      k = (e >> 1) ? n2 - 1 : 0; j = (e & 1) ? n1 - 1 : 0; i = 1 + r - e * ni; mask = 6;
-    }
-    coarse_robin(G, su, srho, i, j, k, mask);
-  }
-  __syncthreads();
-  if (threadIdx.x < 8)
-    coarse_robin(G, su, srho, (threadIdx.x >> 1) & 1 ? n0 - 1 : 0, (threadIdx.x >> 2) & 1 ? n1 - 1 : 0,
-                 threadIdx.x & 1 ? n2 - 1 : 0, 7);
-  __syncthreads();
   for (int q = threadIdx.x; q < np; q += NT) st<double>(ug, unsigned(q) * 8u, su[q]);
   if (threadIdx.x == 0) {
     *It.norm = (unsigned long long)__double_as_longlong(cur);
@@ -3593,31 +3670,37 @@ void launch_ghost_fill(hipStream_t s, const PtBlock *blocks, int nblocks, int or
   }
 }
 
-// coarse-solve shape by box size: up to 2048 points of a colour, 1024
-// threads with 2 points each and their coefficients in registers (512
-// threads with 4 each for the scalar-field and EM equations, whose longer
-// update would spill at 1024 threads); up to 4096 (the 21^3 coarsest box
-// of N=161), 1024 threads with 4 each
+// coarse-solve shape by box size: up to 2048 points of a colour and a shell
+// that the threads hold, 1024 threads with 2 points each and their
+// coefficients in registers (512 threads with 4 each for EM, whose longer
+// update would spill at 1024 threads; the scalar field's 17^3 753 us with 512
+// threads, 598 with 1024); up to 4096 (the 21^3 coarsest box of N=161), 1024
+// threads with 4 each.  Every cube of up to 4096 points of a colour has a
+// shell of at most 3 * 1024 points.
 bool launch_coarse_solve(hipStream_t s, const CoarseItem *items, int n, int max_pts, int max_int,
-                         int eq, double eps, int max_iter) {
+                         int max_shell, int eq, double eps, int max_iter) {
   const size_t lds = 2 * sizeof(double) * size_t(max_pts);  // max_pts: largest B.size
   // max_int: largest number of points of one colour slot list, ceil(ni/2) nj nk
-  if (lds + 2048 > size_t(kLdsLimit) || max_int > 4096) return false;
+  // max_shell: largest number of face and edge points
+  if (lds + 2048 > size_t(kLdsLimit) || max_int > 4096 || max_shell > 3 * 1024) return false;
   if (n == 0) return true;
-  const bool small = max_int <= 2048;
-  const bool wide = eq != 1 && eq != kEqPuncturesEm;
+  const bool em = eq == kEqPuncturesEm;
+  const bool small = max_int <= 2048 && max_shell <= (em ? 3 * 512 : 2 * 1024);
 #define OLL_COARSE(E)                                                                              \
-  if (small && wide)                                                                               \
+  if (small)                                                                                       \
     hipLaunchKernelGGL((k_coarse_solve<E, 2, 1024, 2>), dim3(n), dim3(1024), lds, s, items, eps, max_iter); \
-  else if (small)                                                                                  \
-    hipLaunchKernelGGL((k_coarse_solve<E, 4, 512, 3>), dim3(n), dim3(512), lds, s, items, eps, max_iter); \
   else                                                                                             \
     hipLaunchKernelGGL((k_coarse_solve<E, 4, 1024, 3>), dim3(n), dim3(1024), lds, s, items, eps, max_iter);
   switch (eq) {
     case 1: OLL_COARSE(1) break;
     case 2: OLL_COARSE(2) break;
     case 3: OLL_COARSE(3) break;
-    case kEqPuncturesEm: OLL_COARSE(kEqPuncturesEm) break;
+    case kEqPuncturesEm:
+      if (small)
+        hipLaunchKernelGGL((k_coarse_solve<kEqPuncturesEm, 4, 512, 3>), dim3(n), dim3(512), lds, s, items, eps, max_iter);
+      else
+        hipLaunchKernelGGL((k_coarse_solve<kEqPuncturesEm, 4, 1024, 3>), dim3(n), dim3(1024), lds, s, items, eps, max_iter);
+      break;
     default: OLL_COARSE(0) break;
   }
 #undef OLL_COARSE
@@ -3654,12 +3737,12 @@ void launch_zero_lists(hipStream_t s, const ZeroItem *items, int n) {
 void kernels_init() {
   static bool done = false;
   if (done) return;
-#define OLL_COARSE_FNS(E)                                          \
-  reinterpret_cast<const void *>(&k_coarse_solve<E, 4, 512, 3>),      \
-      reinterpret_cast<const void *>(&k_coarse_solve<E, 2, 1024, 2>), \
+#define OLL_COARSE_FNS(E)                                               \
+  reinterpret_cast<const void *>(&k_coarse_solve<E, 2, 1024, 2>), \
       reinterpret_cast<const void *>(&k_coarse_solve<E, 4, 1024, 3>)
   const void *fns[] = {OLL_COARSE_FNS(0), OLL_COARSE_FNS(1), OLL_COARSE_FNS(2), OLL_COARSE_FNS(3),
-                       OLL_COARSE_FNS(kEqPuncturesEm)};
+                       reinterpret_cast<const void *>(&k_coarse_solve<kEqPuncturesEm, 4, 512, 3>),
+                       reinterpret_cast<const void *>(&k_coarse_solve<kEqPuncturesEm, 4, 1024, 3>)};
 #undef OLL_COARSE_FNS
   for (const void *f : fns)
     (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsLimit - 1024);

@@ -394,6 +394,11 @@ constexpr int kNormWords = kNormSubSlots * kNormStride;  // u64 words per logica
 inline long long coarse_colour_slots(const int n[3]) {
   return (long long)((n[0] - 1) / 2) * (n[1] - 2) * (n[2] - 2);
 }
+// its face and edge points
+inline long long coarse_shell_points(const int n[3]) {
+  const long long ni = n[0] - 2, nj = n[1] - 2, nk = n[2] - 2;
+  return 2 * (nj * nk + ni * nk + ni * nj) + 4 * (ni + nj + nk);
+}
 // largest coarsest box the LDS-resident solve (512 threads) takes: <= 8
 // points per colour per thread, edge points <= 512, u and rho within the LDS
 inline bool coarse_box_fits(const int n[3], long long size) {
@@ -486,7 +491,7 @@ void launch_prolong(hipStream_t s, const PtBlock *blocks, int nblocks);
 void launch_ghost_fill(hipStream_t s, const PtBlock *blocks, int nblocks, int order, int columns);
 // false when the largest box does not fit the LDS-resident kernel
 bool launch_coarse_solve(hipStream_t s, const CoarseItem *items, int n, int max_pts, int max_int,
-                         int eq, double eps, int max_iter);
+                         int max_shell, int eq, double eps, int max_iter);
 void launch_zero_u64(hipStream_t s, unsigned long long *p, long long n);
 // words to clear at one address (each member's own count: the arrays differ)
 struct ZeroItem {
