@@ -1167,11 +1167,20 @@ __device__ __forceinline__ int shell_index(int q, int hi, int n, int R) {
   return hi ? n - R + q : R - 1 - q;
 }
 
-// The corners' Robin updates form one chain per corner (each point reads
-// the ones updated before it), so they run from LDS: the whole block stages
-// each corner's cube of kCornerW^3 points (R <= 4 shell layers plus the 4
-// inward points the one-sided derivatives read) and rho of its R^3 points,
-// eight threads walk the chains, and the updated points are written back.
+// Edges and corners: a point's one-sided derivatives read points further
+// inwards on its axes, so in the reference's order (inwards points first) a
+// point reads exactly the updated values of those shell points, and points
+// whose distances inwards have the same sum are independent of each other.
+// One lane takes a point and the sums go from the innermost outwards: 2R - 1
+// steps for an edge's cross-section instead of R^2, 3R - 2 for a corner
+// instead of R^3, from values staged in LDS, with what does not depend on u
+// formed before the first step.  The chains of dependent divisions, and a
+// staging whose loads waited for each other, bounded both: N=129 8th order
+// edges 24 -> 6.2 us, corners 17 -> 8.6; N=161 6th order 14.2 -> 5.9, 11.0 ->
+// 7.0; one N=65 request 10.6 -> 5.9, 7.8 -> 6.6.
+//
+// A corner's cube has kCornerW^3 points (R <= 4 shell layers plus the 4
+// inward points the derivatives read).
 constexpr int kCornerR = 4;
 constexpr int kCornerW = kCornerR + 4;
 constexpr int kCornerCube = kCornerW * kCornerW * kCornerW;
@@ -1180,148 +1189,27 @@ constexpr int kCornerR3 = kCornerR * kCornerR * kCornerR;
 // box index of local coordinate l (counted inwards from side h) along an axis
 __device__ __forceinline__ int corner_index(int l, int h, int n) { return h ? n - 1 - l : l; }
 
-// one Robin update of corner point (li, lj, lk) (local, counted inwards)
-// of the cube cu of corner (hx, hy, hz): robin_point's arithmetic, with the
-// derivatives' inward neighbours read from the cube
-__device__ __forceinline__ void robin_corner_update(const DevBox &B, double *cu, double rho, int hx,
-                                                    int hy, int hz, int li, int lj, int lk) {
-  const int l[3] = {li, lj, lk}, h[3] = {hx, hy, hz};
-  const int st[3] = {1, kCornerW, kCornerW * kCornerW};
-  const int q = (lk * kCornerW + lj) * kCornerW + li;
-  double X[3];
-  for (int a = 0; a < 3; ++a) X[a] = coord(B, a, corner_index(l[a], h[a], B.n[a]));
-  const double r2 = X[0] * X[0] + X[1] * X[1] + X[2] * X[2];
-  double sF = 0.0, sdF = 0.0;
-  const double u0 = cu[q];
-  for (int a = 0; a < 3; ++a) {
-    const double id = B.idx[a];
-    const double *w = cu + q;
-    const int m = st[a];
-    double cf, dv;
-    // deriv(): dx2 at the box faces for order 2, the one-sided dx4 otherwise
-    if (B.order == 2) {
-      if (!h[a]) {
-        cf = -3.0 * 0.5 * id;
-        dv = (-3.0 * u0 + 4.0 * w[m] - w[2 * m]) * 0.5 * id;
-      } else {
-        cf = 3.0 * 0.5 * id;
-        dv = (3.0 * u0 - 4.0 * w[m] + w[2 * m]) * 0.5 * id;
-      }
-    } else if (!h[a]) {
-      cf = -25.0 * id / 12.0;
-      dv = -(25.0 * u0 - 48.0 * w[m] + 36.0 * w[2 * m] - 16.0 * w[3 * m] + 3.0 * w[4 * m]) * id / 12.0;
-    } else {
-      cf = 25.0 * id / 12.0;
-      dv = (25.0 * u0 - 48.0 * w[m] + 36.0 * w[2 * m] - 16.0 * w[3 * m] + 3.0 * w[4 * m]) * id / 12.0;
-    }
-    sF += dv / X[a];
-    sdF += cf / X[a];
-  }
-  const double op = r2 * B.ipn * sF + u0;
-  const double Fv = op - rho;
-  const double dF = r2 * B.ipn * sdF + 1.0;
-  cu[q] = u0 - Fv / dF;
+// deriv()'s one-sided derivative at side h from the staged point w[0] and the
+// points w[m], w[2 m].. inwards: dx2 at the box faces for order 2, dx4
+// otherwise; cf: the coefficient of the point itself
+__device__ __forceinline__ double inward_deriv(const double *w, int m, int order, int h, double id) {
+  const double u0 = w[0];
+  if (order == 2)
+    return h ? (3.0 * u0 - 4.0 * w[m] + w[2 * m]) * 0.5 * id : (-3.0 * u0 + 4.0 * w[m] - w[2 * m]) * 0.5 * id;
+  const double d = 25.0 * u0 - 48.0 * w[m] + 36.0 * w[2 * m] - 16.0 * w[3 * m] + 3.0 * w[4 * m];
+  return h ? d * id / 12.0 : -d * id / 12.0;
+}
+__device__ __forceinline__ double inward_coef(int order, int h, double id) {
+  const double cf = order == 2 ? 3.0 * 0.5 * id : 25.0 * id / 12.0;
+  return h ? cf : -cf;
 }
 
-// One edge cross-section's Robin updates in the reference's order (outer
-// axis A, inner axis B, both counted inwards from the shell's sides), from
-// registers: the L-shaped set of points its one-sided derivatives read (the
-// R x R shell points and the 4 inward points along A and along B of each)
-// is loaded first, the R^2 updates chain through the registers with
-// robin_point's arithmetic, and the updated points are written back.
-// axa, axb: axes A and B; ha, hb: their sides; e_idx: the index along the
-// edge's own axis (the third).
-template <int R>
-__device__ void robin_edge_chain(const DevBox &B, BoxData D, int axa, int axb, int ha, int hb,
-                                 int e_idx) {
-  constexpr int W = R + 4;
-  double va[R][W];  // local A < R: every local B
-  double vb[4][R];  // local A >= R: local B < R
-  double rho[R][R];
-  // box indices of local point (la, lb)
-  auto index = [&](int la, int lb, int &i, int &j, int &k) {
-    const int pa = ha ? B.n[axa] - 1 - la : la, pb = hb ? B.n[axb] - 1 - lb : lb;
-    i = axa == 0 ? pa : (axb == 0 ? pb : e_idx);
-    j = axa == 1 ? pa : (axb == 1 ? pb : e_idx);
-    k = axa == 2 ? pa : (axb == 2 ? pb : e_idx);
-  };
-#pragma unroll
-  for (int la = 0; la < W; ++la)
-#pragma unroll
-    for (int lb = 0; lb < W; ++lb) {
-      if (la >= R && lb >= R) continue;
-      int i, j, k;
-      index(la, lb, i, j, k);
-      const long long p = pidx(B, i, j, k);
-      if (la < R) va[la][lb] = D.u[p]; else vb[la - R][lb] = D.u[p];
-      if (la < R && lb < R) rho[la][lb] = D.rho[p];
-    }
-  // robin_point takes the masked axes in ascending order
-  const bool a_first = axa < axb;
-#pragma unroll
-  for (int qa = 0; qa < R; ++qa)
-#pragma unroll
-    for (int qb = 0; qb < R; ++qb) {
-      const int la = R - 1 - qa, lb = R - 1 - qb;
-      int i, j, k;
-      index(la, lb, i, j, k);
-      const double X[3] = {coord(B, 0, i), coord(B, 1, j), coord(B, 2, k)};
-      const double r2 = X[0] * X[0] + X[1] * X[1] + X[2] * X[2];
-      double sF = 0.0, sdF = 0.0;
-      const double u0 = va[la][lb];
-#pragma unroll
-      for (int o = 0; o < 2; ++o) {
-        const bool along_a = a_first == (o == 0);
-        // the 4 inward points along the axis (la + m < W, lb + m < W)
-        double w[5];
-        w[0] = u0;
-#pragma unroll
-        for (int m = 1; m <= 4; ++m)
-          w[m] = along_a ? (la + m < R ? va[la + m][lb] : vb[la + m - R][lb]) : va[la][lb + m];
-        const int a = along_a ? axa : axb;
-        const int hs = along_a ? ha : hb;
-        const double id = B.idx[a];
-        const double xa = a == 0 ? X[0] : (a == 1 ? X[1] : X[2]);
-        double cf, dv;
-        if (B.order == 2) {
-          if (!hs) {
-            cf = -3.0 * 0.5 * id;
-            dv = (-3.0 * u0 + 4.0 * w[1] - w[2]) * 0.5 * id;
-          } else {
-            cf = 3.0 * 0.5 * id;
-            dv = (3.0 * u0 - 4.0 * w[1] + w[2]) * 0.5 * id;
-          }
-        } else if (!hs) {
-          cf = -25.0 * id / 12.0;
-          dv = -(25.0 * u0 - 48.0 * w[1] + 36.0 * w[2] - 16.0 * w[3] + 3.0 * w[4]) * id / 12.0;
-        } else {
-          cf = 25.0 * id / 12.0;
-          dv = (25.0 * u0 - 48.0 * w[1] + 36.0 * w[2] - 16.0 * w[3] + 3.0 * w[4]) * id / 12.0;
-        }
-        sF += dv / xa;
-        sdF += cf / xa;
-      }
-      const double op = r2 * B.ipn * sF + u0;
-      const double Fv = op - rho[la][lb];
-      const double dF = r2 * B.ipn * sdF + 1.0;
-      va[la][lb] = u0 - Fv / dF;
-    }
-#pragma unroll
-  for (int la = 0; la < R; ++la)
-#pragma unroll
-    for (int lb = 0; lb < R; ++lb) {
-      int i, j, k;
-      index(la, lb, i, j, k);
-      D.u[pidx(B, i, j, k)] = va[la][lb];
-    }
-}
-
-// Edge cross-section t of a box (faces must be done): its R x R shell
-// points in the reference's order.  Edges XY(4) run along z, XZ(4) along
-// y, YZ(4) along x; within an edge the cross-section is visited outer axis
-// first (x before y for XY, x before z for XZ, z before y for YZ), as
-// Fix_Points orders them.
-__device__ void robin_edge_section(const DevBox &B, BoxData D, int mode, int t) {
+// Edge cross-section t of a box (faces must be done): its R x R shell points
+// by the section's kEdgeLanes lanes, lane q its own.  Edges XY(4) run along
+// z, XZ(4) along y, YZ(4) along x; axis A is x, x, z and B is y, z, y, as
+// Fix_Points orders them.  win: the section's kCornerW^2 staged points.
+constexpr int kEdgeLanes = 16;
+__device__ void robin_edge_section(const DevBox &B, BoxData D, int mode, int t, int q, double *win) {
   const int R = B.R;
   const int nint[3] = {B.n[0] - 2 * R, B.n[1] - 2 * R, B.n[2] - 2 * R};
   int grp, e, s;
@@ -1334,40 +1222,67 @@ __device__ void robin_edge_section(const DevBox &B, BoxData D, int mode, int t) 
     e = (t - 4 * (nint[2] + nint[1])) / nint[0];
     s = (t - 4 * (nint[2] + nint[1])) % nint[0];
   }
-  const int hA = (e >> 1) & 1, hB = e & 1;
-  if (mode == ROBIN_UPDATE && R <= 3) {
-    // outer axis A and inner axis B of the cross-section and their sides
-    // (the orders below); 8th-order boxes (R = 4) would not fit the
-    // registers and take the point-by-point path
-    const int axa = grp == 2 ? 2 : 0, axb = grp == 1 ? 2 : 1;
-    const int ha = grp == 2 ? hB : hA, hb = grp == 2 ? hA : hB;
-    if (R == 1)
-      robin_edge_chain<1>(B, D, axa, axb, ha, hb, R + s);
-    else if (R == 2)
-      robin_edge_chain<2>(B, D, axa, axb, ha, hb, R + s);
-    else
-      robin_edge_chain<3>(B, D, axa, axb, ha, hb, R + s);
+  const int axa = grp == 2 ? 2 : 0, axb = grp == 1 ? 2 : 1;
+  const int h1 = (e >> 1) & 1, h2 = e & 1;
+  const int ha = grp == 2 ? h2 : h1, hb = grp == 2 ? h1 : h2;
+  const int na = B.n[axa], nb = B.n[axb];
+  // box indices of local point (la, lb), counted inwards from the sides
+  auto index = [&](int la, int lb, int &i, int &j, int &k) {
+    const int pa = corner_index(la, ha, na), pb = corner_index(lb, hb, nb);
+    i = axa == 0 ? pa : R + s;
+    j = axb == 1 ? pb : R + s;
+    k = axa == 2 ? pa : (axb == 2 ? pb : R + s);
+  };
+  const bool mine = q < R * R;
+  const int la = mine ? q / R : 0, lb = mine ? q - la * R : 0;
+  int i, j, k;
+  index(la, lb, i, j, k);
+  if (mode != ROBIN_UPDATE) {  // u stays: every point at once
+    if (mine) robin_point(B, D, i, j, k, (1 << axa) | (1 << axb), mode);
     return;
   }
-  for (int qa = 0; qa < R; ++qa)
-    for (int qb = 0; qb < R; ++qb) {
-      int i, j, k, mask;
-      if (grp == 0) {  // XiYi, XiYf, XfYi, XfYf: x outer, y inner; along z
-        i = shell_index(qa, hA, B.n[0], R); j = shell_index(qb, hB, B.n[1], R); k = R + s; mask = 3;
-      } else if (grp == 1) {  // XiZi, XiZf, XfZi, XfZf: x outer, z inner; along y
-        i = shell_index(qa, hA, B.n[0], R); k = shell_index(qb, hB, B.n[2], R); j = R + s; mask = 5;
-      } else {  // YiZi, YiZf, YfZi, YfZf: z outer, y inner; along x
-        j = shell_index(qb, hA, B.n[1], R); k = shell_index(qa, hB, B.n[2], R); i = R + s; mask = 6;
-      }
-      robin_point(B, D, i, j, k, mask, mode);
-    }
+  // all of the square, so that no load waits for a test (what lies beyond the
+  // derivatives' reach is not read)
+#pragma unroll
+  for (int m = 0; m < kCornerW * kCornerW / kEdgeLanes; ++m) {
+    const int l = q + m * kEdgeLanes, wa = l / kCornerW, wb = l % kCornerW;
+    int wi, wj, wk;
+    index(min(wa, na - 1), min(wb, nb - 1), wi, wj, wk);
+    win[l] = D.u[pidx(B, wi, wj, wk)];
+  }
+  const long long p = pidx(B, i, j, k);
+  const double rho = D.rho[p];
+  const double X[3] = {coord(B, 0, i), coord(B, 1, j), coord(B, 2, k)};
+  const double r2n = (X[0] * X[0] + X[1] * X[1] + X[2] * X[2]) * B.ipn;
+  // the two axes in ascending order, as robin_point takes them
+  const bool a_first = axa < axb;
+  const int ax1 = a_first ? axa : axb, ax2 = a_first ? axb : axa;
+  const int s1 = a_first ? ha : hb, s2 = a_first ? hb : ha;
+  const int m1 = a_first ? kCornerW : 1, m2 = a_first ? 1 : kCornerW;
+  const double id1 = B.idx[ax1], id2 = B.idx[ax2];
+  const double x1 = ax1 == 0 ? X[0] : X[1], x2 = ax2 == 1 ? X[1] : X[2];
+  const double dF = r2n * (inward_coef(B.order, s1, id1) / x1 + inward_coef(B.order, s2, id2) / x2) + 1.0;
+  double *w = win + la * kCornerW + lb;
+#pragma unroll 1
+  for (int sum = 2 * (kCornerR - 1); sum >= 0; --sum) {
+    // the section's lanes lie in one wave, whose LDS accesses keep their
+    // order: only the compiler has to
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_wave_barrier();
+    if (!mine || la + lb != sum) continue;
+    const double u0 = w[0];
+    const double sF =
+        0.0 + inward_deriv(w, m1, B.order, s1, id1) / x1 + inward_deriv(w, m2, B.order, s2, id2) / x2;
+    const double un = u0 - (r2n * sF + u0 - rho) / dF;
+    w[0] = un;
+    D.u[p] = un;
+  }
 }
 
 // corners of one box, by one block (edges must be done): k outer, j, i
 // inner (domain.cc:592-695); corner c has hz = bit 0, hx = bit 1, hy = bit
-// 2.  cube and crho: 8 kCornerCube and 8 kCornerR3 doubles of LDS, for the
-// corner chains (R <= kCornerR)
-__device__ void robin_corners(const DevBox &B, BoxData D, int mode, double *cube, double *crho) {
+// 2.  cube: 8 kCornerCube doubles of LDS; corner c is wave c's, a lane a point
+__device__ void robin_corners(const DevBox &B, BoxData D, int mode, double *cube) {
   const int R = B.R;
   if (mode != ROBIN_UPDATE) {
     // the operator modes leave u alone: every corner point at once
@@ -1381,43 +1296,55 @@ __device__ void robin_corners(const DevBox &B, BoxData D, int mode, double *cube
     }
     return;
   }
-  // stage the eight cubes (points beyond a small box are never read) and
-  // the corner points' rho
-  for (int t = threadIdx.x; t < 8 * kCornerCube; t += blockDim.x) {
-    const int c = t / kCornerCube, q = t - c * kCornerCube;
-    const int hz = c & 1, hx = (c >> 1) & 1, hy = (c >> 2) & 1;
-    const int li = q % kCornerW, lj = (q / kCornerW) % kCornerW, lk = q / (kCornerW * kCornerW);
-    double v = 0.0;
-    if (li < B.n[0] && lj < B.n[1] && lk < B.n[2]) {
-      const long long p = pidx(B, corner_index(li, hx, B.n[0]), corner_index(lj, hy, B.n[1]),
-                               corner_index(lk, hz, B.n[2]));
-      v = D.u[p];
-      if (li < R && lj < R && lk < R) crho[c * kCornerR3 + (lk * kCornerR + lj) * kCornerR + li] = D.rho[p];
+  const int c = int(threadIdx.x) / kCornerR3, q = int(threadIdx.x) % kCornerR3;
+  const bool mine = q < R * R * R;
+  const int lk = mine ? q / (R * R) : 0, lj = mine ? (q / R) % R : 0, li = mine ? q % R : 0;
+  const int l[3] = {li, lj, lk}, h[3] = {(c >> 1) & 1, (c >> 2) & 1, c & 1};
+  const int ijk[3] = {corner_index(li, h[0], B.n[0]), corner_index(lj, h[1], B.n[1]),
+                      corner_index(lk, h[2], B.n[2])};
+  double X[3];
+  for (int a = 0; a < 3; ++a) X[a] = coord(B, a, ijk[a]);
+  const double r2n = (X[0] * X[0] + X[1] * X[1] + X[2] * X[2]) * B.ipn;
+  double sdF = 0.0;
+  for (int a = 0; a < 3; ++a) sdF += inward_coef(B.order, h[a], B.idx[a]) / X[a];
+  const double dF = r2n * sdF + 1.0;
+  double *w = cube + c * kCornerCube + (lk * kCornerW + lj) * kCornerW + li;
+  const int st[3] = {1, kCornerW, kCornerW * kCornerW};
+  // a point stages itself and, if it is the shell's innermost on an axis, the
+  // points inwards of it; every lane loads them (within the box) at once
+  const long long p = pidx(B, ijk[0], ijk[1], ijk[2]);
+  const double rho = D.rho[p], own = D.u[p];
+  const int reach = B.order == 2 ? 2 : 4;
+  double in[3][4];
+#pragma unroll
+  for (int a = 0; a < 3; ++a)
+#pragma unroll
+    for (int m = 1; m <= 4; ++m) {
+      int at[3] = {ijk[0], ijk[1], ijk[2]};
+      at[a] = corner_index(min(l[a] + m, B.n[a] - 1), h[a], B.n[a]);
+      in[a][m - 1] = D.u[pidx(B, at[0], at[1], at[2])];
     }
-    cube[t] = v;
+  if (mine) {
+    w[0] = own;
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+#pragma unroll
+      for (int m = 1; m <= 4; ++m)
+        if (l[a] == R - 1 && m <= reach) w[m * st[a]] = in[a][m - 1];
   }
-  __syncthreads();
-  if (threadIdx.x < 8) {
-    const int c = threadIdx.x;
-    const int hz = c & 1, hx = (c >> 1) & 1, hy = (c >> 2) & 1;
-    double *cu = cube + c * kCornerCube;
-    const double *cr = crho + c * kCornerR3;
-    // shell_index(q, h, n, R) is local coordinate R - 1 - q from either side
-    for (int qk = 0; qk < R; ++qk)
-      for (int qj = 0; qj < R; ++qj)
-        for (int qi = 0; qi < R; ++qi) {
-          const int li = R - 1 - qi, lj = R - 1 - qj, lk = R - 1 - qk;
-          robin_corner_update(B, cu, cr[(lk * kCornerR + lj) * kCornerR + li], hx, hy, hz, li, lj, lk);
-        }
-  }
-  __syncthreads();
-  const int R3 = R * R * R;
-  for (int t = threadIdx.x; t < 8 * R3; t += blockDim.x) {
-    const int c = t / R3, q = t - c * R3;
-    const int hz = c & 1, hx = (c >> 1) & 1, hy = (c >> 2) & 1;
-    const int lk = q / (R * R), lj = (q / R) % R, li = q % R;
-    D.u[pidx(B, corner_index(li, hx, B.n[0]), corner_index(lj, hy, B.n[1]), corner_index(lk, hz, B.n[2]))] =
-        cube[c * kCornerCube + (lk * kCornerW + lj) * kCornerW + li];
+#pragma unroll 1
+  for (int sum = 3 * (R - 1); sum >= 0; --sum) {
+    // one wave, as for the edges
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_wave_barrier();
+    if (!mine || l[0] + l[1] + l[2] != sum) continue;
+    double sF = 0.0;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) sF += inward_deriv(w, st[a], B.order, h[a], B.idx[a]) / X[a];
+    const double u0 = w[0];
+    const double un = u0 - (r2n * sF + u0 - rho) / dF;
+    w[0] = un;
+    D.u[p] = un;
   }
 }
 
@@ -1435,12 +1362,13 @@ __global__ __launch_bounds__(256) void k_robin_faces(const RobinItem *__restrict
   robin_face_column(B, box_data(B), g - items[lo].col0, mode);
 }
 
-// edges: one thread per (box, edge cross-section), spread over many
-// workgroups (a box's edges are a chain of R^2 dependent updates each)
-constexpr int kRobinEdgeThreads = 128;
+// edges: kEdgeLanes lanes per (box, edge cross-section)
+constexpr int kRobinEdgeThreads = 256, kEdgeSections = kRobinEdgeThreads / kEdgeLanes;
 __global__ __launch_bounds__(kRobinEdgeThreads) void k_robin_edges(const RobinItem *__restrict__ items,
                                                                    int n, int total, int mode) {
-  const int g = blockIdx.x * blockDim.x + threadIdx.x;
+  __shared__ double win[kEdgeSections][kCornerW * kCornerW + 2];
+  const int sec = int(threadIdx.x) / kEdgeLanes, q = int(threadIdx.x) % kEdgeLanes;
+  const int g = int(blockIdx.x) * kEdgeSections + sec;
   if (g >= total) return;
   int lo = 0, hi = n - 1;
   while (lo < hi) {
@@ -1448,15 +1376,15 @@ __global__ __launch_bounds__(kRobinEdgeThreads) void k_robin_edges(const RobinIt
     if (items[mid].ecol0 <= g) lo = mid; else hi = mid - 1;
   }
   const DevBox &B = *items[lo].box;
-  robin_edge_section(B, box_data(B), mode, g - items[lo].ecol0);
+  robin_edge_section(B, box_data(B), mode, g - items[lo].ecol0, q, win[sec]);
 }
 
 // corners: one block per box
-__global__ __launch_bounds__(512) void k_robin_corners(const RobinItem *__restrict__ items,
+__global__ __launch_bounds__(8 * kCornerR3) void k_robin_corners(const RobinItem *__restrict__ items,
                                                        int mode) {
-  __shared__ double cube[8 * kCornerCube], crho[8 * kCornerR3];
+  __shared__ double cube[8 * kCornerCube];
   const DevBox &B = *items[blockIdx.x].box;
-  robin_corners(B, box_data(B), mode, cube, crho);
+  robin_corners(B, box_data(B), mode, cube);
 }
 
 // Robin operator value at a shell point (no update)
@@ -3618,9 +3546,9 @@ void launch_robin(hipStream_t s, const RobinItem *items, int n, int total_cols, 
   if (n == 0) return;
   hipLaunchKernelGGL(k_robin_faces, dim3(ceil_div(total_cols, 256)), dim3(256), 0, s, items, n,
                      total_cols, mode);
-  hipLaunchKernelGGL(k_robin_edges, dim3(ceil_div(total_edges, kRobinEdgeThreads)),
+  hipLaunchKernelGGL(k_robin_edges, dim3(ceil_div(total_edges, kEdgeSections)),
                      dim3(kRobinEdgeThreads), 0, s, items, n, total_edges, mode);
-  hipLaunchKernelGGL(k_robin_corners, dim3(n), dim3(512), 0, s, items, mode);
+  hipLaunchKernelGGL(k_robin_corners, dim3(n), dim3(8 * kCornerR3), 0, s, items, mode);
 }
 
 void launch_restrict_u(hipStream_t s, const PtBlock *blocks, int nblocks) {

@@ -178,3 +178,18 @@ def test_paired_operator(eq, n, order):
                 assert np.abs(a - b).max() <= 1e-5 * np.abs(b - u0).max(), (lv, ib)
     m.close()
     h.close()
+
+
+@pytest.mark.parametrize("order", [2, 4, 6, 8])
+@pytest.mark.parametrize("n", [25, 41])
+def test_robin_shell(n, order):
+    """The Robin update of faces, edges and corners, one to four shell layers
+    deep, on the smallest boxes and beside larger ones."""
+    h, s = pair(argv(0, n, order))
+    seed_state(h, s, 17)
+    for lv in range(s.mgrid + 1):
+        h.robin(lv)
+        for ib in s.level_boxes(lv):
+            s.robin(ib)
+            assert rel_err(h.get_field(ib, oa.F_U), s.field(ib, O.F_U)) < 1e-12, (lv, ib)
+    h.close()
