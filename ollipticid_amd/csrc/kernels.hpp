@@ -399,8 +399,8 @@ inline long long coarse_shell_points(const int n[3]) {
   const long long ni = n[0] - 2, nj = n[1] - 2, nk = n[2] - 2;
   return 2 * (nj * nk + ni * nk + ni * nj) + 4 * (ni + nj + nk);
 }
-// largest coarsest box the LDS-resident solve (512 threads) takes: <= 8
-// points per colour per thread, edge points <= 512, u and rho within the LDS
+// largest coarsest box the LDS-resident solve takes: at most 4096
+// points of a colour, edge points <= 512, u and rho within the LDS
 inline bool coarse_box_fits(const int n[3], long long size) {
   const long long ni = n[0] - 2, nj = n[1] - 2, nk = n[2] - 2;
   return coarse_colour_slots(n) <= 8 * 512 && 4 * (ni + nj + nk) <= 512 &&
