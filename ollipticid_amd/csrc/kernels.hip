@@ -469,12 +469,6 @@ __device__ __forceinline__ bool row_slot(const RowBlock &Bk, ConstBox &B, unsign
   return true;
 }
 
-// the larger of acc and a, a NaN in either kept (one step from acc = 0
-// gives a itself, NaN included)
-__device__ __forceinline__ double nan_max(double acc, double a) {
-  return (a > acc || !(a == a)) ? a : acc;
-}
-
 // a whole-row block's rows, rpb = blockDim / per_row at a time: f(rpb,
 // lr0) for the first local row lr0 of each chunk (blocks of one launch
 // over many requests hold several chunks)
@@ -886,7 +880,9 @@ __device__ __forceinline__ bool row_pair(const RowBlock &Bk, ConstBox &B, unsign
 }
 
 // operator on the interior: mode RES_OPERATOR r = N(u), RES_DEFECT
-// w = rho - N(u), RES_DERIVATIVE r = dN/du_p; the norm is max |N(u)|
+// w = rho - N(u), RES_DERIVATIVE r = dN/du_p; the norm is max |N(u)| over
+// the points where N(u) is a number (fmax drops a NaN, which must not reach
+// wave_norm: as a bit pattern it would outrank its wave's other points)
 template <int ORD, int EQ>
 __global__ __launch_bounds__(kRowThreads) void k_residual(const RowBlock *__restrict__ blocks,
                                                           unsigned per_row, float inv_per_row,
@@ -917,7 +913,7 @@ __global__ __launch_bounds__(kRowThreads) void k_residual(const RowBlock *__rest
 #pragma unroll
       for (int q = 0; q < 2; ++q) {
         v[q] = mode == RES_DEFECT ? rho[q] - N[q] : (mode == RES_DERIVATIVE ? dN[q] : N[q]);
-        if (ok[q]) rmax = nan_max(rmax, fabs(N[q]));
+        if (ok[q]) rmax = fmax(rmax, fabs(N[q]));
       }
       if (ok[0] && ok[1])
         st_pair(out, o, v[0], v[1]);
@@ -941,7 +937,7 @@ __global__ __launch_bounds__(kRowThreads) void k_residual(const RowBlock *__rest
       st<double>(B.f[F_W], o, rho - N);
     else
       st<double>(B.f[F_R], o, mode == RES_DERIVATIVE ? dN : N);
-    rmax = nan_max(rmax, fabs(N));
+    rmax = fmax(rmax, fabs(N));
   });
   wave_norm(Bk.norm, rmax, seen);
 }
@@ -985,7 +981,7 @@ __global__ __launch_bounds__(kRowThreads) void k_defect32(const RowBlock *__rest
       st<float>(B.g[G_R], o4, float(res));
       st<float>(B.g[G_Q], o4, float(dN[q] - B.dulap));
       st<float>(B.g[G_E], o4, 0.0f);
-      rmax = nan_max(rmax, fabs(res));
+      rmax = fmax(rmax, fabs(res));
       if (!(res == res)) rmax = __longlong_as_double(0x7ff0000000000000LL);
     }
   });
