@@ -342,7 +342,9 @@ int oll_engine_kernel_launches(oll_engine *e, int cap, double *bytes, double *ms
 /* Launch-shape table (no reference counterpart; filled by the autotuner,
  * ollipticid_amd/autotune.py): threads per workgroup of the smoothers'
  * colour passes for one precision (OLL_PREC_*) and order, a multiple of 64
- * from 64 to 512 (default 256; raised to hold one interior row).
+ * from 64 to 512, raised to hold one interior row.  256, the default, leaves
+ * launches of few points to smaller workgroups (64 or 128 by the launch's
+ * length); any other size holds for every launch.
  * Process-wide; schedules built afterwards use it.  Results do not depend
  * on it.  The setter returns OLL_EINVAL for other values. */
 int oll_set_sweep_threads(int precision, int order, int threads);

@@ -6,8 +6,9 @@ binary workload at that order (N=65, 9 levels, nu2=20; the engine's
 per-launch HIP events, launches issued one by one) with every candidate
 workgroup size, twice: as a batch of requests and as one request alone
 (the launches of a lightly loaded server).  The rate of each is the
-algorithmic bytes of the updated points over the passes' device time.  A
-size replaces the 256-thread default only when it is faster than the
+algorithmic bytes of the updated points over the passes' device time.  256
+threads is the default, with which launches of few points take 64 or 128; the
+other candidates hold for every launch.  A size replaces the default only when it is faster than the
 default in both regimes by at least MIN_GAIN; of those, the one whose worse
 regime gains most.  The colour passes' results do not depend on the size:
 the tuner only changes speed.  It writes ollipticid_amd/launch_shapes.json, which the

@@ -757,8 +757,9 @@ struct Builder {
       std::vector<RowBlock> cb, sb;
       double bytes[5] = {0, 0, 0, 0, 0};
       std::set<const DevBox *> boxes;
-      // colour-pass workgroup size from the launch-shape table and the
-      // launch's length, at least one interior row
+      // colour-pass workgroup size from the launch-shape table (and the
+      // launch's length, where the table holds the default), at least one
+      // interior row
       long long nthreads = 0;
       for (int h : g.second) {
         const Hier &H = *M[size_t(h)];
@@ -766,7 +767,7 @@ struct Builder {
         for (int b = f; b < f + n; ++b)
           nthreads += (long long)interior_rows(H.hbox[size_t(b)]) * row_threads(H.hbox[size_t(b)], pts);
       }
-      int threads = std::min(sweep_threads(mixed ? 1 : 0, order), sweep_rule(nthreads));
+      int threads = sweep_size(sweep_threads(mixed ? 1 : 0, order), nthreads);
       while (threads < pc && threads < kMaxRowThreads) threads *= 2;
       int sreps = 1;
       if (mixed) {

@@ -204,9 +204,10 @@ constexpr int sweep_points(int eq) { return eq == kEqPuncturesEm ? 1 : 2; }
 // launch-shape table (sweep_threads); their results do not depend on it
 constexpr int kMaxRowThreads = 512;
 int sweep_threads(int mixed, int order);
-// The table's size is the most a launch takes; launches of few points take
-// smaller workgroups, which spread over more CUs and need no barrier for
-// their norm (64).  Measured, FP64, 64 / 128 / 256 threads: one N=65 4th-order
+// The table's default, kRowThreads, is the most a launch takes: launches of
+// few points take smaller workgroups, which spread over more CUs and need no
+// barrier for their norm (64).  Any other size in the table is a caller's
+// choice and holds for every launch.  Measured, FP64, 64 / 128 / 256 threads: one N=65 4th-order
 // request (46,000 threads a pass) 32.9 / 33.9 / 34.3 ms per 10 V-cycles; one
 // N=129 8th-order box (225,000) 7.5 / 6.4 / 7.7 us a pass; 16 N=65 requests
 // (740,000) 12.7 / 12.9 / 12.6 us; the largest N=161 box (5.4 M) 196 / 196 /
@@ -214,6 +215,10 @@ int sweep_threads(int mixed, int order);
 constexpr int kFewRowThreads = 128;
 constexpr int sweep_rule(long long launch_threads) {
   return launch_threads <= 100000 ? 64 : (launch_threads <= 800000 ? kFewRowThreads : kMaxRowThreads);
+}
+constexpr int sweep_size(int setting, long long launch_threads) {
+  return setting == kRowThreads && sweep_rule(launch_threads) < setting ? sweep_rule(launch_threads)
+                                                                        : setting;
 }
 bool set_sweep_threads(int mixed, int order, int threads);
 
