@@ -707,14 +707,19 @@ __device__ __forceinline__ void smooth_pairs(const RowBlock &Bk, const SweepBox 
 // box1: the one box of every listed block, when the launch covers a single
 // box (else null); its descriptor is then fetched without waiting for the
 // block's.
-// Four waves per SIMD leave a wave the registers to issue its loads (17 at
-// 4th, 25 at 6th, 29 at 8th order) before it waits for the first; compiled
-// for more waves it issued 11 to 14 and waited.  With the scalar loads
-// together (SweepBox): N=161 smoother 94.2 -> 90.3 ms per two V-cycles, 16 x
-// N=65 23.8 -> 23.1, N=129 8th order 21.3 -> 20.4, one 33^3 solve 6.40 ->
-// 6.28.
+// By pairs, four waves per SIMD leave a wave the registers to issue its loads
+// (17 at 4th, 25 at 6th, 29 at 8th order) before it waits for the first;
+// compiled for more waves it issued 11 to 14 and waited.  With the scalar
+// loads together (SweepBox): N=161 smoother 94.2 -> 90.3 ms per two V-cycles,
+// 16 x N=65 23.8 -> 23.1, N=129 8th order 21.3 -> 20.4, one 33^3 solve 6.40 ->
+// 6.28.  Poisson and Brill waves the same way, N=129, a pass before the pairs
+// and now: 2nd order 8.2 -> 6.6 and 6.8 us, 8th 8.5 -> 6.0.  One point a
+// thread (Punctures_EM) has few loads to issue and needs the waves: four a
+// SIMD instead of five to eight took 24.6 us instead of 20.3 (N=129 2nd
+// order), 17.7 instead of 15.4 (4th).
 template <int ORD, int EQ>
-__global__ __launch_bounds__(kMaxRowThreads) __attribute__((amdgpu_waves_per_eu(4, 4)))
+__global__ __launch_bounds__(kMaxRowThreads)
+__attribute__((amdgpu_waves_per_eu(sweep_points(EQ) == 2 ? 4 : 1, sweep_points(EQ) == 2 ? 4 : 8)))
 void k_smooth(const RowBlock *__restrict__ blocks,
                                                         unsigned per_row, float inv_per_row,
                                                         int colour, const DevBox *box1) {
