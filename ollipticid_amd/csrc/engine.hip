@@ -767,7 +767,7 @@ struct Builder {
         for (int b = f; b < f + n; ++b)
           nthreads += (long long)interior_rows(H.hbox[size_t(b)]) * row_threads(H.hbox[size_t(b)], pts);
       }
-      int threads = sweep_size(sweep_threads(mixed ? 1 : 0, order), nthreads);
+      int threads = sweep_size(sweep_threads(mixed ? 1 : 0, order), nthreads, mixed, pts);
       while (threads < pc && threads < kMaxRowThreads) threads *= 2;
       int sreps = 1;
       if (mixed) {

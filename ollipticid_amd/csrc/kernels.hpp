@@ -207,18 +207,33 @@ int sweep_threads(int mixed, int order);
 // The table's default, kRowThreads, is the most a launch takes: launches of
 // few points take smaller workgroups, which spread over more CUs and need no
 // barrier for their norm (64).  Any other size in the table is a caller's
-// choice and holds for every launch.  Measured, FP64, 64 / 128 / 256 threads: one N=65 4th-order
-// request (46,000 threads a pass) 32.9 / 33.9 / 34.3 ms per 10 V-cycles; one
-// N=129 8th-order box (225,000) 7.5 / 6.4 / 7.7 us a pass; 16 N=65 requests
-// (740,000) 12.7 / 12.9 / 12.6 us; the largest N=161 box (5.4 M) 196 / 196 /
-// 193 us.
+// choice and holds for every launch.  The limits, in threads a launch, with
+// us a pass (top level, events) and ms per two V-cycles of one box with 64 /
+// 128 / 256 threads:
+//   FP64 by pairs, 64 up to 100,000 and 128 up to 800,000: 71,000 (N=97 8th
+//     order) 4.4 / 4.4 / 4.5 and 3.22 / 3.24 / 3.41; 190,000 (N=129 8th)
+//     6.2 / 6.1 / 7.0, 4.66 / 4.63 / 4.82; 516,000 (N=129 2nd) 6.6 / 6.9 /
+//     7.4, 3.51 / 3.53 / 3.58; 736,000 (N=145 2nd) 12.7 / 10.8 / 11.2, 5.10 /
+//     4.95 / 4.99; the largest N=161 box (5.4 M) 196 / 196 / 193 us.
+//   FP64 one point a thread, 64 up to 200,000: 164,000 (N=97 4th) 6.2 / 7.0 /
+//     6.7 and 4.66 / 4.77 / 4.70; 391,000 (N=129 4th) 12.1 / 12.1 / 11.7,
+//     8.94 / 8.97 / 8.86.
+//   FP32 (no norm), 64 up to 100,000 and 128 up to 300,000: 39,000 (N=65 8th)
+//     4.24 each and 3.07 / 3.07 / 3.07; 154,000 (N=81 4th) 4.28 each, 4.71 /
+//     4.69 / 4.81; 366,000 (N=129 8th) 4.8 / 4.6 / 4.4, 4.26 / 4.27 / 4.20;
+//     676,000 (N=145 6th) 6.9 / 5.0 / 4.5, 5.49 / 5.17 / 5.08.
 constexpr int kFewRowThreads = 128;
-constexpr int sweep_rule(long long launch_threads) {
-  return launch_threads <= 100000 ? 64 : (launch_threads <= 800000 ? kFewRowThreads : kMaxRowThreads);
+constexpr int sweep_rule(long long launch_threads, bool mixed, int pts) {
+  const bool one = !mixed && pts == 1;
+  if (launch_threads <= (one ? 200000 : 100000)) return 64;
+  if (launch_threads <= (mixed ? 300000 : (one ? 0 : 800000))) return kFewRowThreads;
+  return kMaxRowThreads;
 }
-constexpr int sweep_size(int setting, long long launch_threads) {
-  return setting == kRowThreads && sweep_rule(launch_threads) < setting ? sweep_rule(launch_threads)
-                                                                        : setting;
+// the table's size `setting` for a launch of launch_threads threads of pts
+// points each
+constexpr int sweep_size(int setting, long long launch_threads, bool mixed, int pts) {
+  const int most = sweep_rule(launch_threads, mixed, pts);
+  return setting == kRowThreads && most < setting ? most : setting;
 }
 bool set_sweep_threads(int mixed, int order, int threads);
 

@@ -11,16 +11,25 @@ namespace {
 // a size set by the caller holds for every launch; the default leaves
 // launches of few threads to smaller workgroups and never a larger one
 int check_sweep_size() {
-  const long long lengths[] = {1, 1000, 99999, 100001, 500000, 5000000, 1LL << 33};
-  for (long long n : lengths) {
-    for (int set = 64; set <= kMaxRowThreads; set += 64)
-      if (set != kRowThreads && sweep_size(set, n) != set)
-        return std::printf("sweep_size(%d, %lld) = %d\n", set, n, sweep_size(set, n)), 1;
-    const int d = sweep_size(kRowThreads, n);
-    if (d > kRowThreads || d < 64 || d % 64 != 0 || (n <= 1000 && d != 64) ||
-        (n >= 5000000 && d != kRowThreads))
-      return std::printf("sweep_size(default, %lld) = %d\n", n, d), 1;
-  }
+  // threads a launch -> the default's workgroup: pairs, one point a thread, FP32
+  const struct {
+    long long n;
+    int pairs, one, fp32;
+  } want[] = {{1, 64, 64, 64},           {100000, 64, 64, 64},
+              {100001, 128, 64, 128},    {200000, 128, 64, 128},
+              {200001, 128, 256, 128},   {300000, 128, 256, 128},
+              {300001, 128, 256, 256},   {800000, 128, 256, 256},
+              {800001, 256, 256, 256},   {1LL << 33, 256, 256, 256}};
+  for (const auto &w : want)
+    for (int kind = 0; kind < 3; ++kind) {
+      const bool mixed = kind == 2;
+      const int pts = kind == 0 ? 2 : 1, d = kind == 0 ? w.pairs : (kind == 1 ? w.one : w.fp32);
+      for (int set = 64; set <= kMaxRowThreads; set += 64) {
+        const int got = sweep_size(set, w.n, mixed, pts);
+        if (got != (set == kRowThreads ? d : set))
+          return std::printf("sweep_size(%d, %lld, %d, %d) = %d\n", set, w.n, mixed, pts, got), 1;
+      }
+    }
   return 0;
 }
 
