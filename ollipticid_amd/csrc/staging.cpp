@@ -4,7 +4,6 @@
 #include <cstring>
 #include <mutex>
 #include <new>
-#include <system_error>
 #include <thread>
 
 namespace oll {
@@ -85,7 +84,7 @@ void host_copy(void *dst, const void *src, size_t bytes) {
         th[started] = std::thread([d, s, b, share] { std::memcpy(d + b, s + b, share); });
         begin += share;
       }
-    } catch (const std::system_error &) {  // no thread to be had: the rest here
+    } catch (...) {  // no thread or no memory for one: the rest here
     }
   }
   std::memcpy(d + begin, s + begin, bytes - begin);
