@@ -6,6 +6,8 @@
 #include <cmath>
 #include <cstring>
 #include <map>
+#include <memory>
+#include <new>
 #include <set>
 #include <tuple>
 
@@ -1567,6 +1569,34 @@ struct StagingUse {
   }
 };
 
+// field_host without pinned memory: the colour blocks whole, through pageable
+// memory, reordered by the host
+static int field_pageable(const DevBox &b, hipStream_t s, int field, double *host, bool to_host,
+                          std::string &err) {
+  const std::unique_ptr<double[]> st(new (std::nothrow) double[size_t(b.size)]());
+  if (!st) return err = "host memory for a field", OLL_ENOMEM;
+  const size_t bytes = size_t(b.size) * sizeof(double);
+  if (to_host) {
+    ENG_CHECK(hipMemcpyAsync(st.get(), b.f[field], bytes, hipMemcpyDeviceToHost, s));
+    ENG_CHECK(hipStreamSynchronize(s));
+  }
+  size_t q = 0;
+  for (int k = 0; k < b.n[2]; ++k)
+    for (int j = 0; j < b.n[1]; ++j)
+      for (int i = 0; i < b.n[0]; ++i, ++q) {
+        double &v = st[size_t(pidx(b, i, j, k))];
+        if (to_host)
+          host[q] = v;
+        else
+          v = host[q];
+      }
+  if (!to_host) {
+    ENG_CHECK(hipMemcpyAsync(b.f[field], st.get(), bytes, hipMemcpyHostToDevice, s));
+    ENG_CHECK(hipStreamSynchronize(s));
+  }
+  return OLL_OK;
+}
+
 // One half of the staging is filled or drained by the GPU while the host
 // copies the other: fields of one half's size take one launch and one copy
 int field_host(Hier &H, hipStream_t s, int ibox, int field, double *host, bool to_host,
@@ -1575,7 +1605,7 @@ int field_host(Hier &H, hipStream_t s, int ibox, int field, double *host, bool t
   const size_t np = size_t(npts(b)), half = Staging::kBytes / sizeof(double);
   const size_t chunks = (np + half - 1) / half;
   StagingUse use(s);
-  if (!use.g) return err = "pinned staging memory", OLL_ENOMEM;
+  if (!use.g) return field_pageable(b, s, field, host, to_host, err);
   if (chunks > 1) ENG_CHECK(use.events());
   auto begin = [&](size_t c) { return c * half; };
   auto count = [&](size_t c) { return std::min(half, np - c * half); };
@@ -1604,6 +1634,25 @@ int field_host(Hier &H, hipStream_t s, int ibox, int field, double *host, bool t
   return OLL_OK;
 }
 
+// interp_points without pinned memory
+static int interp_pageable(Hier &H, hipStream_t s, int field, int npts, const int *box,
+                           const double *xyz, int ord, double *out, std::string &err) {
+  int *d_box = nullptr;
+  double *d_xyz = nullptr, *d_out = nullptr;
+  TempBuffers tmp;
+  const size_t n = size_t(npts);
+  ENG_CHECK(tmp.alloc(&d_box, n));
+  ENG_CHECK(tmp.alloc(&d_xyz, 3 * n));
+  ENG_CHECK(tmp.alloc(&d_out, n));
+  ENG_CHECK(hipMemcpyAsync(d_box, box, n * sizeof(int), hipMemcpyHostToDevice, s));
+  ENG_CHECK(hipMemcpyAsync(d_xyz, xyz, 3 * n * sizeof(double), hipMemcpyHostToDevice, s));
+  launch_interp_points(s, H.dbox, field, d_box, d_xyz, npts, ord, d_out);
+  ENG_CHECK(hipGetLastError());
+  ENG_CHECK(hipMemcpyAsync(out, d_out, n * sizeof(double), hipMemcpyDeviceToHost, s));
+  ENG_CHECK(hipStreamSynchronize(s));
+  return OLL_OK;
+}
+
 int interp_points(Hier &H, hipStream_t s, int field, int npts, const int *box, const double *xyz,
                   int ord, double *out, std::string &err) {
   if (npts <= 0) return OLL_OK;
@@ -1620,12 +1669,12 @@ int interp_points(Hier &H, hipStream_t s, int field, int npts, const int *box, c
   const size_t half = n <= kSplit ? n : std::min(kMost, (n + 127) / 128 * 64);
   const size_t chunks = (n + half - 1) / half;
   const bool direct = n <= kFew;
+  StagingUse use(s);
+  if (!use.g) return interp_pageable(H, s, field, npts, box, xyz, ord, out, err);
   if (!direct && !H.interp_scratch) {
     ENG_CHECK(hipMalloc(reinterpret_cast<void **>(&H.interp_scratch), kMost * kIn));
     H.bytes += kMost * kIn;
   }
-  StagingUse use(s);
-  if (!use.g) return err = "pinned staging memory", OLL_ENOMEM;
   if (chunks > 1) ENG_CHECK(use.events());
   for (size_t c = 0; c <= chunks; ++c) {
     if (c < chunks) {

@@ -26,6 +26,8 @@ void destroy(Staging *s) {
 }
 }  // namespace
 
+hipError_t (*staging_malloc)(void **, size_t, unsigned) = hipHostMalloc;
+
 Staging *staging_take() {
   {
     std::lock_guard<std::mutex> lock(g_mu);
@@ -34,7 +36,8 @@ Staging *staging_take() {
   Staging *s = new (std::nothrow) Staging();
   if (!s) return nullptr;
   for (char *&p : s->half)
-    if (hipHostMalloc(reinterpret_cast<void **>(&p), Staging::kBytes, hipHostMallocPortable) != hipSuccess) {
+    if (staging_malloc(reinterpret_cast<void **>(&p), Staging::kBytes, hipHostMallocPortable) != hipSuccess) {
+      (void)hipGetLastError();  // no later check reports it
       p = nullptr;
       destroy(s);
       return nullptr;

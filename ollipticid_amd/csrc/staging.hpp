@@ -18,8 +18,11 @@ struct Staging {
   char *half[2] = {nullptr, nullptr};
 };
 
-// null when the memory cannot be had
+// null when the memory cannot be had: callers then go without (pageable
+// copies, slower)
 Staging *staging_take();
+// hipHostMalloc; tests put a failing one in its place
+extern hipError_t (*staging_malloc)(void **, size_t, unsigned);
 void staging_give(Staging *s);
 // a handle begins or ends
 void staging_retain();
