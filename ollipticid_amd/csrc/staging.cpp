@@ -9,7 +9,7 @@
 namespace oll {
 
 namespace {
-constexpr int kKeep = 4;
+constexpr int kKeep = 16;
 constexpr int kCopyThreads = 4;
 constexpr size_t kThreadBytes = size_t(256) << 10;  // least share of a thread
 
@@ -49,7 +49,7 @@ void staging_give(Staging *s) {
   if (!s) return;
   {
     std::lock_guard<std::mutex> lock(g_mu);
-    if (g_handles > 0 && g_nidle < kKeep) {
+    if (g_nidle < kKeep && g_nidle < g_handles) {
       g_idle[g_nidle++] = s;
       return;
     }

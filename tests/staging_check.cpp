@@ -1,6 +1,7 @@
 // Host check of ollipticid_amd/csrc/staging.cpp with the HIP calls replaced:
 // copies that cannot start their threads.  Prints "ok" and exits 0, or what
 // fails and exits 1.
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <new>
@@ -17,13 +18,17 @@ void *operator new(std::size_t n) {
 void operator delete(void *p) noexcept { std::free(p); }
 void operator delete(void *p, std::size_t) noexcept { std::free(p); }
 
+static int g_held = 0, g_mallocs = 0;  // buffers not freed, allocations so far
 hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
   *p = std::malloc(n);
+  ++g_held;
+  ++g_mallocs;
   return *p ? hipSuccess : hipErrorOutOfMemory;
 }
 hipError_t hipGetLastError() { return hipSuccess; }
 hipError_t hipHostFree(void *p) {
   std::free(p);
+  --g_held;
   return hipSuccess;
 }
 
@@ -48,10 +53,38 @@ int check_copy() {
   return 0;
 }
 
+// `callers` calls at once over `handles` handles: the second round allocates
+// only what the bound (16, and one a handle) keeps from staying, and nothing
+// is left with the last handle
+int check_pool() {
+  for (int handles : {1, 4, 16, 40})
+    for (int callers : {1, 4, 5, 16, 24}) {
+      const int kept = std::min(16, std::min(handles, callers));
+      for (int h = 0; h < handles; ++h) oll::staging_retain();
+      int fresh = 0;
+      for (int round = 0; round < 2; ++round) {
+        const int before = g_mallocs;
+        std::vector<oll::Staging *> use;
+        for (int c = 0; c < callers; ++c) {
+          use.push_back(oll::staging_take());
+          if (!use.back()) return std::printf("no staging\n"), 1;
+        }
+        for (oll::Staging *s : use) oll::staging_give(s);
+        fresh = g_mallocs - before;
+      }
+      if (fresh != 2 * (callers - kept) || g_held != 2 * kept)
+        return std::printf("%d handles, %d callers: %d allocated again, %d held\n", handles, callers,
+                           fresh, g_held), 1;
+      for (int h = 0; h < handles; ++h) oll::staging_release();
+      if (g_held != 0) return std::printf("%d buffers left\n", g_held), 1;
+    }
+  return 0;
+}
+
 }  // namespace
 
 int main() {
-  if (check_copy()) return 1;
+  if (check_copy() || check_pool()) return 1;
   std::puts("ok");
   return 0;
 }
