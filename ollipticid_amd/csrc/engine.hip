@@ -1551,9 +1551,10 @@ void puncture_approx(const Hier &H, double *u_at_p) {
 // a borrowed Staging, returned on every path once the stream is done with it
 struct StagingUse {
   hipStream_t s;
-  Staging *g = staging_take();
+  Staging *g;
   hipEvent_t ev[2] = {nullptr, nullptr};
-  explicit StagingUse(hipStream_t stream) : s(stream) {}
+  // chunks: pieces of the call; two halves where there are several
+  StagingUse(hipStream_t stream, size_t chunks) : s(stream), g(staging_take(chunks > 1 ? 2 : 1)) {}
   ~StagingUse() {
     (void)hipStreamSynchronize(s);
     for (hipEvent_t e : ev)
@@ -1604,7 +1605,7 @@ int field_host(Hier &H, hipStream_t s, int ibox, int field, double *host, bool t
   const DevBox &b = H.hbox[size_t(ibox)];
   const size_t np = size_t(npts(b)), half = Staging::kBytes / sizeof(double);
   const size_t chunks = (np + half - 1) / half;
-  StagingUse use(s);
+  StagingUse use(s, chunks);
   if (!use.g) return field_pageable(b, s, field, host, to_host, err);
   if (chunks > 1) ENG_CHECK(use.events());
   auto begin = [&](size_t c) { return c * half; };
@@ -1669,7 +1670,7 @@ int interp_points(Hier &H, hipStream_t s, int field, int npts, const int *box, c
   const size_t half = n <= kSplit ? n : std::min(kMost, (n + 127) / 128 * 64);
   const size_t chunks = (n + half - 1) / half;
   const bool direct = n <= kFew;
-  StagingUse use(s);
+  StagingUse use(s, chunks);
   if (!use.g) return interp_pageable(H, s, field, npts, box, xyz, ord, out, err);
   if (!direct && !H.interp_scratch) {
     ENG_CHECK(hipMalloc(reinterpret_cast<void **>(&H.interp_scratch), kMost * kIn));

@@ -28,20 +28,22 @@ void destroy(Staging *s) {
 
 hipError_t (*staging_malloc)(void **, size_t, unsigned) = hipHostMalloc;
 
-Staging *staging_take() {
+Staging *staging_take(int halves) {
+  Staging *s = nullptr;
   {
     std::lock_guard<std::mutex> lock(g_mu);
-    if (g_nidle > 0) return g_idle[--g_nidle];
+    if (g_nidle > 0) s = g_idle[--g_nidle];
   }
-  Staging *s = new (std::nothrow) Staging();
-  if (!s) return nullptr;
-  for (char *&p : s->half)
-    if (staging_malloc(reinterpret_cast<void **>(&p), Staging::kBytes, hipHostMallocPortable) != hipSuccess) {
+  if (!s && !(s = new (std::nothrow) Staging())) return nullptr;
+  for (int i = 0; i < halves; ++i) {
+    char *&p = s->half[i];
+    if (!p && staging_malloc(reinterpret_cast<void **>(&p), Staging::kBytes, hipHostMallocPortable) != hipSuccess) {
       (void)hipGetLastError();  // no later check reports it
       p = nullptr;
       destroy(s);
       return nullptr;
     }
+  }
   return s;
 }
 
@@ -67,8 +69,8 @@ void staging_release() {
   int n = 0;
   {
     std::lock_guard<std::mutex> lock(g_mu);
-    if (--g_handles > 0) return;
-    while (g_nidle > 0) drop[n++] = g_idle[--g_nidle];
+    --g_handles;
+    while (g_nidle > g_handles) drop[n++] = g_idle[--g_nidle];
   }
   while (n > 0) destroy(drop[--n]);
 }

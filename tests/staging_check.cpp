@@ -54,9 +54,9 @@ int check_copy() {
 }
 
 // `callers` calls at once over `handles` handles: the second round allocates
-// only what the bound (16, and one a handle) keeps from staying, and nothing
-// is left with the last handle
-int check_pool() {
+// only what the bound (16, and one a handle) keeps from staying, and no more
+// is left than there are handles
+int check_pool(int halves) {
   for (int handles : {1, 4, 16, 40})
     for (int callers : {1, 4, 5, 16, 24}) {
       const int kept = std::min(16, std::min(handles, callers));
@@ -66,25 +66,49 @@ int check_pool() {
         const int before = g_mallocs;
         std::vector<oll::Staging *> use;
         for (int c = 0; c < callers; ++c) {
-          use.push_back(oll::staging_take());
-          if (!use.back()) return std::printf("no staging\n"), 1;
+          use.push_back(oll::staging_take(halves));
+          if (!use.back() || !use.back()->half[halves - 1]) return std::printf("no staging\n"), 1;
         }
         for (oll::Staging *s : use) oll::staging_give(s);
         fresh = g_mallocs - before;
       }
-      if (fresh != 2 * (callers - kept) || g_held != 2 * kept)
+      if (fresh != halves * (callers - kept) || g_held != halves * kept)
         return std::printf("%d handles, %d callers: %d allocated again, %d held\n", handles, callers,
                            fresh, g_held), 1;
-      for (int h = 0; h < handles; ++h) oll::staging_release();
-      if (g_held != 0) return std::printf("%d buffers left\n", g_held), 1;
+      for (int h = handles - 1; h >= 0; --h) {
+        oll::staging_release();
+        if (g_held != halves * std::min(h, kept))
+          return std::printf("%d buffers left with %d handles\n", g_held, h), 1;
+      }
     }
+  return 0;
+}
+
+// one half, then both of the same, and nothing where the second cannot be had
+int check_halves() {
+  oll::staging_retain();
+  oll::Staging *s = oll::staging_take(1);
+  if (!s || g_held != 1) return std::printf("one half: %d held\n", g_held), 1;
+  oll::staging_give(s);
+  oll::Staging *t = oll::staging_take(2);
+  if (t != s || g_held != 2) return std::printf("both halves: %d held\n", g_held), 1;
+  oll::staging_give(t);
+  oll::Staging *u = oll::staging_take(1), *v = oll::staging_take(1);
+  if (u != s || g_held != 3) return std::printf("a second: %d held\n", g_held), 1;
+  oll::staging_give(v);
+  oll::staging_malloc = [](void **, size_t, unsigned) { return hipErrorOutOfMemory; };
+  if (oll::staging_take(2) || g_held != 2) return std::printf("no memory: %d held\n", g_held), 1;
+  oll::staging_malloc = hipHostMalloc;
+  oll::staging_give(u);
+  oll::staging_release();
+  if (g_held != 0) return std::printf("%d buffers left\n", g_held), 1;
   return 0;
 }
 
 }  // namespace
 
 int main() {
-  if (check_copy() || check_pool()) return 1;
+  if (check_copy() || check_pool(1) || check_pool(2) || check_halves()) return 1;
   std::puts("ok");
   return 0;
 }

@@ -16,8 +16,8 @@ class NoPinned:
 
     def __enter__(self):
         self.L = oa.load()
-        self.take = getattr(self.L, "_ZN3oll12staging_takeEv")
-        self.take.restype, self.take.argtypes = C.c_void_p, []
+        self.take = getattr(self.L, "_ZN3oll12staging_takeEi")
+        self.take.restype, self.take.argtypes = C.c_void_p, [C.c_int]
         self.give = getattr(self.L, "_ZN3oll12staging_giveEPNS_7StagingE")
         self.give.restype, self.give.argtypes = None, [C.c_void_p]
         self.hook = C.c_void_p.in_dll(self.L, "_ZN3oll14staging_mallocE")
@@ -32,7 +32,7 @@ class NoPinned:
         self.hook.value = C.cast(self.fail, C.c_void_p).value
         self.held = []
         while True:
-            s = self.take()
+            s = self.take(1)
             if not s:
                 break
             self.held.append(s)
