@@ -600,8 +600,9 @@ int oll_engine_admit_hier(oll_engine *e, oll_hier *h, long long tag) {
   if (!e || !h) return fail(OLL_EINVAL, "null argument");
   if (!h->H.slab) return fail(OLL_EINVAL, "empty hierarchy handle");
   if (h->H.prob.method != OLL_METHOD_VCYCLE) return fail(OLL_EINVAL, "the engine runs V-cycle requests");
-  if (e->budget && e->in_use + h->H.bytes > e->budget) return fail(OLL_EBUSY, "HBM budget exhausted");
   CAPI_CHECK(hipStreamSynchronize(h->stream));
+  hier_drop_scratch(h->H);  // no part of what the budget is to hold
+  if (e->budget && e->in_use + h->H.bytes > e->budget) return fail(OLL_EBUSY, "HBM budget exhausted");
   release_schedule(h->vcycle);
   release_schedule(h->scratch);
   oll_engine::Member m;

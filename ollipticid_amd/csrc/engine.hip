@@ -472,6 +472,18 @@ int hier_reset(Hier &H, hipStream_t s, std::string &err) {
   return OLL_OK;
 }
 
+// a chunk of interp_points: coordinates, box and value of a point, and the
+// points of one half of the staging
+static constexpr size_t kInterpIn = 3 * sizeof(double) + sizeof(int);
+static constexpr size_t kInterpMost = Staging::kBytes / (kInterpIn + sizeof(double)) / 64 * 64;
+
+void hier_drop_scratch(Hier &H) {
+  if (!H.interp_scratch) return;
+  (void)hipFree(H.interp_scratch);
+  H.interp_scratch = nullptr;
+  H.bytes -= kInterpMost * kInterpIn;
+}
+
 void hier_release(Hier &H) {
   (void)hipFree(H.slab);
   (void)hipFree(H.slab32);
@@ -482,8 +494,7 @@ void hier_release(Hier &H) {
   (void)hipFree(H.dxfer);
   (void)hipFree(H.norms);
   (void)hipFree(H.iters);
-  (void)hipFree(H.interp_scratch);
-  H.interp_scratch = nullptr;
+  hier_drop_scratch(H);
   H.slab = nullptr;
   H.slab32 = nullptr;
   H.dbox = nullptr;
@@ -1663,8 +1674,7 @@ int interp_points(Hier &H, hipStream_t s, int field, int npts, const int *box, c
   // pinned half and reads few points from it; many are first copied to the
   // handle's device scratch, which the chunks share on the stream (reading
   // 28 bytes a point over PCIe would take longer than interpolating).
-  constexpr size_t kIn = 3 * sizeof(double) + sizeof(int), kPoint = kIn + sizeof(double);
-  constexpr size_t kMost = Staging::kBytes / kPoint / 64 * 64;
+  constexpr size_t kIn = kInterpIn, kMost = kInterpMost;
   constexpr size_t kFew = 4096, kSplit = 65536;
   const size_t n = size_t(npts);
   const size_t half = n <= kSplit ? n : std::min(kMost, (n + 127) / 128 * 64);

@@ -83,6 +83,8 @@ struct Hier {
 // coefficients; returns an OLL_* code and sets err
 int hier_build(Hier &H, const oll_problem &p, hipStream_t s, std::string &err);
 void hier_release(Hier &H);
+// frees what calls keep on the hierarchy for later ones (interp_scratch)
+void hier_drop_scratch(Hier &H);
 // per colour pass, the points of level l inside their boxes' rho boxes
 std::vector<double> level_rho_points(const Hier &H, int l);
 // boxes first .. first + count - 1 read rho everywhere from now on (after a

@@ -67,3 +67,26 @@ def test_exchange_without_pinned_memory(n, order):
             assert no.calls >= 6  # every call went without
             assert h.residual(h.levels - 1) >= 0.0  # no error is left behind
         assert np.array_equal(h.get_field(ib, oa.F_V), a)
+
+
+def test_point_calls_leave_the_budget_alone():
+    """A hierarchy that fills an engine's budget is admitted again after a
+    call of many points on it."""
+    p = oa.problem_from_argv(argv(0, 25, 2))
+    p.max_cycles = 2
+    h = oa.Hierarchy(p)
+    built = h.device_bytes()
+    e = oa.Engine(hbm_budget=built)
+    try:
+        for tag in (1, 2):
+            assert e.admit_hier(h, tag), tag
+            while e.step():
+                pass
+            (_, _, _, h), = e.pop_hier({tag: p})
+            b = h.boxes()[-1]
+            xyz = np.random.default_rng(3).uniform(b["origin"], b["end"], (5000, 3))
+            h.interp(oa.F_U, np.full(5000, h.nbox - 1), xyz, 4)
+            assert h.device_bytes() >= built
+        assert e.admit_hier(h, 3)
+    finally:
+        e.close()
