@@ -1186,7 +1186,7 @@ int build_vcycle_from(const std::vector<Hier *> &M, const std::vector<int> &star
   for (Hier *H : M) {
     const DevBox &B = H->hbox[size_t(H->geo.level_first[0])];
     if (!coarse_box_fits(B.n, B.size))
-      return err = "coarsest box exceeds the LDS of one workgroup", OLL_EINVAL;
+      return err = "coarsest box too large for one workgroup (points, shell points or LDS)", OLL_EINVAL;
     // k_coarse_solve's Robin shell and sweeps are those of a 2nd-order box
     if (B.nc != 2 || B.R != 1) return err = "coarsest box must be 2nd order", OLL_EINVAL;
   }
@@ -1326,7 +1326,7 @@ int issue(const Schedule &S, hipStream_t s, Timing *t, std::string &err) {
       case Launch::COARSE:
         if (!launch_coarse_solve(s, reinterpret_cast<const CoarseItem *>(items), L.n, L.max_pts,
                                  L.max_int, L.max_row, L.eq, 2 * DBL_EPSILON, 100000))
-          return err = "coarsest box exceeds the LDS of one workgroup", OLL_EINVAL;
+          return err = "coarsest box too large for one workgroup (points, shell points or LDS)", OLL_EINVAL;
         break;
       case Launch::CORR_V:
         launch_corr_v(s, reinterpret_cast<const PtBlock *>(items), L.n);

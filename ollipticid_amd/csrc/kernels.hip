@@ -3412,7 +3412,6 @@ void restrict_defect_impl(hipStream_t s, const PtBlock *blocks, int nb) {
   hipLaunchKernelGGL((k_restrict_defect<ORD, EQ>), dim3(nb), dim3(kPtThreads), 0, s, blocks);
 }
 
-constexpr int kLdsLimit = 160 * 1024;
 
 }  // namespace
 
@@ -3611,7 +3610,8 @@ bool launch_coarse_solve(hipStream_t s, const CoarseItem *items, int n, int max_
   const size_t lds = 2 * sizeof(double) * size_t(max_pts);  // max_pts: largest B.size
   // max_int: largest number of points of one colour slot list, ceil(ni/2) nj nk
   // max_shell: largest number of face and edge points
-  if (lds + 2048 > size_t(kLdsLimit) || max_int > 4096 || max_shell > 3 * 1024) return false;
+  if (lds > size_t(kCoarseMostLds) || max_int > kCoarseMostSlots || max_shell > kCoarseMostShell)
+    return false;
   if (n == 0) return true;
   const bool em = eq == kEqPuncturesEm;
   const bool small = max_int <= 2048 && max_shell <= (em ? 3 * 512 : 2 * 1024);
@@ -3674,7 +3674,7 @@ void kernels_init() {
                        reinterpret_cast<const void *>(&k_coarse_solve<kEqPuncturesEm, 4, 1024, 3>)};
 #undef OLL_COARSE_FNS
   for (const void *f : fns)
-    (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsLimit - 1024);
+    (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, kCoarseMostLds);
   done = true;
 }
 

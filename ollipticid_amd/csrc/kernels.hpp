@@ -419,12 +419,14 @@ inline long long coarse_shell_points(const int n[3]) {
   const long long ni = n[0] - 2, nj = n[1] - 2, nk = n[2] - 2;
   return 2 * (nj * nk + ni * nk + ni * nj) + 4 * (ni + nj + nk);
 }
-// largest coarsest box the LDS-resident solve takes: at most 4096
-// points of a colour, edge points <= 512, u and rho within the LDS
+// largest coarsest box the LDS-resident solve takes (k_coarse_solve's shapes):
+// points of a colour, face and edge points, edge points, bytes of u and rho
+constexpr int kCoarseMostSlots = 4096, kCoarseMostShell = 3 * 1024, kCoarseMostEdges = 512;
+constexpr int kCoarseMostLds = 160 * 1024 - 2048;
 inline bool coarse_box_fits(const int n[3], long long size) {
   const long long ni = n[0] - 2, nj = n[1] - 2, nk = n[2] - 2;
-  return coarse_colour_slots(n) <= 8 * 512 && 4 * (ni + nj + nk) <= 512 &&
-         2 * 8 * size + 2048 <= 160 * 1024;
+  return coarse_colour_slots(n) <= kCoarseMostSlots && coarse_shell_points(n) <= kCoarseMostShell &&
+         4 * (ni + nj + nk) <= kCoarseMostEdges && 2 * 8 * size <= kCoarseMostLds;
 }
 
 void launch_coefficients_box(hipStream_t s, const DevBox &B, const PunctureArgs &pa,
@@ -509,7 +511,7 @@ void launch_prolong(hipStream_t s, const PtBlock *blocks, int nblocks);
 // columns = 1: blocks over shell columns (R points across a face slab, one
 // thread each); 0: blocks over shell points
 void launch_ghost_fill(hipStream_t s, const PtBlock *blocks, int nblocks, int order, int columns);
-// false when the largest box does not fit the LDS-resident kernel
+// false when the largest box does not fit the kernel (coarse_box_fits)
 bool launch_coarse_solve(hipStream_t s, const CoarseItem *items, int n, int max_pts, int max_int,
                          int max_shell, int eq, double eps, int max_iter);
 void launch_zero_u64(hipStream_t s, unsigned long long *p, long long n);

@@ -33,10 +33,31 @@ int check_sweep_size() {
   return 0;
 }
 
+// a coarsest box that the schedule builder takes is one that the launcher
+// takes; the cubes are those of up to 21 points an axis
+int check_coarse_box() {
+  for (int a = 3; a <= 131; ++a)
+    for (int b = 3; b <= 131; ++b)
+      for (int c = 3; c <= 131; ++c) {
+        const int n[3] = {a, b, c};
+        const long long size = layout_size(n, 2);
+        const bool fits = coarse_box_fits(n, size);
+        const bool launches = 2 * (long long)sizeof(double) * size <= kCoarseMostLds &&
+                              coarse_colour_slots(n) <= kCoarseMostSlots &&
+                              coarse_shell_points(n) <= kCoarseMostShell &&
+                              4 * ((a - 2) + (b - 2) + (c - 2)) <= kCoarseMostEdges;
+        if (fits != launches || (a == b && b == c && fits != (a <= 21)))
+          return std::printf("box %d x %d x %d: fits %d, launches %d\n", a, b, c, fits, launches), 1;
+      }
+  const int flat[3] = {56, 56, 3};  // 1458 points of a colour, 6484 of the shell
+  if (coarse_box_fits(flat, layout_size(flat, 2))) return std::puts("56 x 56 x 3 fits"), 1;
+  return 0;
+}
+
 }  // namespace
 
 int main() {
-  if (check_sweep_size()) return 1;
+  if (check_sweep_size() || check_coarse_box()) return 1;
   std::puts("ok");
   return 0;
 }
