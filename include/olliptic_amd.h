@@ -360,10 +360,9 @@ int oll_get_sweep_threads(int precision, int order);
 int oll_set_fused_sweeps(int on);
 int oll_get_fused_sweeps(void);
 /* Shared-load transfer kernels (no reference counterpart): on (the
- * default), the ghost-shell fill (elliptic.cc:1905-1908) of boxes of order
- * 6 and 8 runs one thread per column of R shell points across a face slab,
- * loading the interpolation nodes once for the whole column (orders 2 and
- * 4 stay point by point, which measures faster there), and the defect
+ * default), the ghost-shell fill (elliptic.cc:1905-1908) takes the points of
+ * a face in tiles, whose interpolation nodes are loaded once and whose sums
+ * along an axis are formed once for all points that share them, and the defect
  * filter ahead of an off-lattice restriction runs one thread per run of 4
  * points along x, loading the neighbour rows once for the run; off, both
  * go point by point.  The same bits either way.  Process-wide; schedules

@@ -489,10 +489,9 @@ __device__ __forceinline__ Nbr<NC> box_offs(ConstBox &B, int c, int s) {
 
 // ------------------------------------------------------------------
 // smoother: one colour of one Newton-Gauss-Seidel sweep on the rows of
-// every listed block
-// ------------------------------------------------------------------
-// smoother: one colour of one Newton-Gauss-Seidel sweep on the rows of
 // every listed block; thread (lr, t) owns colour point t of local row lr
+// (smooth_rows, Punctures_EM) or points 2t and 2t + 1 (smooth_pairs)
+// ------------------------------------------------------------------
 template <int ORD, int EQ>
 __device__ __forceinline__ void smooth_rows(const RowBlock &Bk, ConstBox &B, unsigned per_row,
                                             float inv_per_row, int colour) {
@@ -2290,7 +2289,7 @@ __global__ __launch_bounds__(kPtThreads) void k_prolong(const PtBlock *__restric
       ConstBox &S = cbox(xs[src].src);
       const void *vf = S.f[F_V];
       const int ex = ext[0], ey = ext[1], ez = ext[2];
-      // rows of the node block, one a quarter wave: ex <= 36 nodes
+      // rows of the node block, one a half wave: ex <= 36 nodes
       for (int r = int(threadIdx.x >> 5); r < ey * ez; r += kPtThreads / 32) {
         const int z = r / ey, y = r - z * ey;
         for (int x = int(threadIdx.x & 31u); x < ex; x += 32)
@@ -2499,7 +2498,7 @@ __global__ __launch_bounds__(kPtThreads) void k_ghost_fill(const PtBlock *__rest
 
 // Ghost shell of refinement boxes by tiles: a workgroup takes kColSuper^2
 // columns of one face side (one block of slots, shell_column), R points
-// each, and interpolates them as one tensor product (tile_interp).  Point by
+// each, and interpolates them as one tensor product (tile_transfer).  Point by
 // point (or column by column) every target summed its own (order + 2)^3
 // nodes.  Measured, per launch: N=129 8th order 400 -> 32 us, N=161 6th
 // order 322 -> 48, 16 x N=65 4th order 146 -> 36.

@@ -181,16 +181,17 @@ struct DevXfer {
 // row-parallel launches: one workgroup per RowBlock, which owns `rows`
 // consecutive rows of one box starting at row0.  For the colour passes
 // (k_smooth, k_smooth32) a row is an interior row (j, k) and a thread owns
-// one colour point of it; for the whole-row kernels (residual, defect,
-// update) a row is the points of one colour of an interior row (one row of
-// that colour's block) and a thread owns one slot of it.
+// one or two adjacent colour points of it (sweep_points; k_smooth32 one); for
+// the whole-row kernels (residual, defect, update) a row is the points of one
+// colour of an interior row (one row of that colour's block) and a thread owns
+// sweep_points adjacent slots of it.
 struct RowBlock {
   const DevBox *box;
   unsigned long long *norm;  // null: no norm
   int row0;
   int rows;
   // segments per row: a row longer than the launch's threads per row is
-  // split into nseg segments of that many slots, each a row of its own in
+  // split into nseg segments of that many threads, each a row of its own in
   // the block numbering (row index = row * nseg + segment)
   int nseg;
 };
@@ -431,9 +432,9 @@ inline bool coarse_box_fits(const int n[3], long long size) {
 
 void launch_coefficients_box(hipStream_t s, const DevBox &B, const PunctureArgs &pa,
                              double robin_a);
-// per_row: threads per row (colour points per interior row for the colour
-// passes, slots per colour row for the whole-row kernels); the host sizes
-// RowBlock::rows to at most kRowThreads / per_row
+// per_row: threads per row (of an interior row's colour points for the colour
+// passes, of a colour row's slots for the whole-row kernels); the host sizes
+// RowBlock::rows to at most the launch's threads / per_row
 // Row kernels address fields with 32-bit byte offsets: a box field must stay
 // below 4 GiB (checked when the hierarchy is built).
 constexpr long long kMaxFieldBytes = 1LL << 32;
@@ -508,8 +509,8 @@ int filter_run_length();
 void launch_corr_v(hipStream_t s, const PtBlock *blocks, int nblocks);
 void launch_prolong(hipStream_t s, const PtBlock *blocks, int nblocks);
 // order: stencil order of the target (refinement) boxes; Lagrange order+1
-// columns = 1: blocks over shell columns (R points across a face slab, one
-// thread each); 0: blocks over shell points
+// columns = 1: blocks over tiles of shell columns (kColSuper^2 columns of R
+// points across a face slab, k_ghost_tiles); 0: blocks over shell points
 void launch_ghost_fill(hipStream_t s, const PtBlock *blocks, int nblocks, int order, int columns);
 // false when the largest box does not fit the kernel (coarse_box_fits)
 bool launch_coarse_solve(hipStream_t s, const CoarseItem *items, int n, int max_pts, int max_int,

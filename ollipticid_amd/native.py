@@ -181,9 +181,9 @@ def fused_sweeps():
 
 
 def set_shared_loads(on):
-    """Ghost fills of 6th- and 8th-order boxes one thread per shell column
-    and defect filters one thread per run of points along x (the default),
-    or both point by point; the same bits either way."""
+    """Ghost fills by tiles of a face's points and defect filters one thread
+    per run of points along x (the default), or both point by point; the same
+    bits either way."""
     _check(load().oll_set_shared_loads(1 if on else 0))
 
 
