@@ -191,7 +191,8 @@ int oll_num_boxes(const oll_hier *h);
 int oll_level_boxes(const oll_hier *h, int level, int *first, int *count);
 int oll_box_info(const oll_hier *h, int ibox, oll_box_desc *out);
 /* Bytes of HBM the hierarchy holds: 3.3 MB more than when it was built once
- * oll_interp has taken more than 4096 points, until an engine admits it. */
+ * oll_interp has taken more than 4096 points, until an engine that has a
+ * budget admits it. */
 size_t oll_device_bytes(const oll_hier *h);
 /* Box table of the hierarchy a problem would build, host only (no device
  * needed): elliptic.cc:300-921 Set_Grids.  Writes min(cap, *nbox) boxes. */

@@ -601,7 +601,10 @@ int oll_engine_admit_hier(oll_engine *e, oll_hier *h, long long tag) {
   if (!h->H.slab) return fail(OLL_EINVAL, "empty hierarchy handle");
   if (h->H.prob.method != OLL_METHOD_VCYCLE) return fail(OLL_EINVAL, "the engine runs V-cycle requests");
   CAPI_CHECK(hipStreamSynchronize(h->stream));
-  hier_drop_scratch(h->H);  // no part of what the budget is to hold
+  // no part of what a budget is to hold; kept without one (freeing it and
+  // allocating it again cost a batch of 16 resident N=65 binaries with points
+  // read back 9 of 291 ms)
+  if (e->budget) hier_drop_scratch(h->H);
   if (e->budget && e->in_use + h->H.bytes > e->budget) return fail(OLL_EBUSY, "HBM budget exhausted");
   release_schedule(h->vcycle);
   release_schedule(h->scratch);
