@@ -559,10 +559,27 @@ int transfer_fields(Hier &H, hipStream_t s, int from, int ffield, int to, int tf
   if (!rc) rc = upload(&dx, xf, bytes, err);
   std::vector<PtBlock> blocks;
   const int mode = (region & 3) | (all ? 4 : 0) | (to_zero ? 8 : 0);
+  long long all_points = 0;
+  for (int t = 0; t < nt; ++t) all_points += npts(H.hbox[size_t(ft + t)]);
+  // Lagrange transfers go by tiles.  A tile of targets coarser than their
+  // source reads more nodes than the LDS holds and is done point by point
+  // within the tile kernel, four points a thread in turn, at two or three waves
+  // per SIMD; it then only pays by its smaller table of blocks, where points are
+  // few (the shell) or cheap.  us a call onto a coarser level, by points / by
+  // tiles: order 2 25^3 92 / 101, 65^3 97 / 98, 113^3 147 / 125; order 3 33^3
+  // 93 / 109, 113^3 172 / 174, 129^3 146 / 139; order 9 33^3 180 / 370, 97^3 406
+  // / 401 and 529 / 714, 129^3 415 / 451 and 396 / 324; the shell, order 9,
+  // 33^3 112 / 117, 65^3 108 / 102, 129^3 145 / 132.
+  const bool few = region == REG_BOUNDARY || nodes == 3;
+  const bool tiles =
+      nodes > 2 && (to >= from || (few && all_points >= (1 << 18)) || (nodes == 4 && all_points >= (1 << 21)));
+  // point by point, from 2^21 points on with four chunks a block (order 9, onto
+  // two levels of N=129: 427 -> 415 us and 592 -> 486; 1.2 M points 700 -> 840)
+  const long long run = kPtThreads * (nodes > 2 && all_points >= (1 << 21) ? 4 : 1);
   for (int t = 0; t < nt; ++t) {
     const DevBox &B = H.hbox[size_t(ft + t)];
     const long long np = npts(B), plane = (long long)B.n[0] * B.n[1];
-    if (nodes > 2) {  // Lagrange: tiles
+    if (tiles) {
       for (int k = 0; k < B.n[2]; k += kXferTile[2])
         for (int j = 0; j < B.n[1]; j += kXferTile[1])
           for (int i = 0; i < B.n[0]; i += kXferTile[0])
@@ -570,13 +587,13 @@ int transfer_fields(Hier &H, hipStream_t s, int from, int ffield, int to, int tf
                                      mode, 0u, 0u, i, j, k});
       continue;
     }
-    for (long long q0 = 0; q0 < np; q0 += kPtThreads)
+    for (long long q0 = 0; q0 < np; q0 += run)
       blocks.push_back(PtBlock{H.dbox + ft + t, dx + refs[size_t(t)].off, refs[size_t(t)].cnt, mode,
-                               unsigned(q0), unsigned(std::min<long long>(kPtThreads, np - q0)),
+                               unsigned(q0), unsigned(std::min<long long>(run, np - q0)),
                                int(q0 % B.n[0]), int((q0 % plane) / B.n[0]), int(q0 / plane)});
   }
   if (!rc) rc = upload(&db, blocks, bytes, err);
-  if (!rc && !launch_transfer_fields(s, db, int(blocks.size()), ffield, tfield, nodes))
+  if (!rc && !launch_transfer_fields(s, db, int(blocks.size()), ffield, tfield, nodes, tiles))
     rc = (err = "unsupported interpolation", OLL_EINVAL);
   if (!rc && hipStreamSynchronize(s) != hipSuccess) rc = (err = "transfer failed", OLL_EDEVICE);
   (void)hipFree(ip);

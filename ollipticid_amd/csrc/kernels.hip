@@ -1889,10 +1889,11 @@ __device__ __forceinline__ void tile_transfer(TileLds<KP> &L, const PtBlock &Bk,
 // (or, with `all` (bit 2), whose extent does); with `to_zero` (bit 3) the
 // last source alone decides and a point it does not hold is set to 0 (the
 // reference's source loop overwrites every point on each pass)
-// Linear transfers go point by point, Lagrange ones by tiles of
-// kXferTile targets (tile_transfer): N=129 8th order, one 135^3 box from its
-// parent, 1175 -> 78 us.
-__global__ __launch_bounds__(kPtThreads) void k_transfer_linear(const PtBlock *__restrict__ blocks,
+// Linear transfers, and most onto a coarser level, go point by point; other
+// Lagrange ones by tiles of kXferTile targets (tile_transfer): N=129 8th order,
+// one 135^3 box from its parent, 1175 -> 78 us.  (transfer_fields has the rule.)
+template <int KP>
+__global__ __launch_bounds__(kPtThreads) void k_transfer_points(const PtBlock *__restrict__ blocks,
                                                                 int ff, int tf) {
   const PtBlock Bk = blocks[xcd_block()];
   ConstBox &T = cbox(Bk.box);
@@ -1912,10 +1913,14 @@ __global__ __launch_bounds__(kPtThreads) void k_transfer_linear(const PtBlock *_
       if ((f & 1) || (all && (f & 2))) {
         ConstBox &S = cbox(X.src);
         double v;
-        if (f & 4)  // a source node: its value (interpolation.cc:140-147)
-          v = ld<double>(S.f[ff], boff(S, X.ax[0].coinc[i], X.ax[1].coinc[j], X.ax[2].coinc[k]));
-        else
-          v = trilinear_field(S, S.f[ff], X, t);
+        if constexpr (KP == 2) {
+          if (f & 4)  // a source node: its value (interpolation.cc:140-147)
+            v = ld<double>(S.f[ff], boff(S, X.ax[0].coinc[i], X.ax[1].coinc[j], X.ax[2].coinc[k]));
+          else
+            v = trilinear_field(S, S.f[ff], X, t);
+        } else {
+          v = tinterp<KP>(S, S.f[ff], X, t, fl);
+        }
         st<double>(T.f[tf], o, v);
         return;
       }
@@ -3636,12 +3641,16 @@ bool launch_coarse_solve(hipStream_t s, const CoarseItem *items, int n, int max_
 }
 
 bool launch_transfer_fields(hipStream_t s, const PtBlock *blocks, int nblocks, int ff, int tf,
-                            int nodes) {
+                            int nodes, bool tiles) {
   if (nblocks == 0) return true;
-#define OLL_TF(KP) hipLaunchKernelGGL(k_transfer_tiles<KP>, dim3(nblocks), dim3(kPtThreads), 0, s, blocks, ff, tf)
+#define OLL_TF(KP)                                                                                     \
+  if (tiles)                                                                                           \
+    hipLaunchKernelGGL(k_transfer_tiles<KP>, dim3(nblocks), dim3(kPtThreads), 0, s, blocks, ff, tf);   \
+  else                                                                                                 \
+    hipLaunchKernelGGL(k_transfer_points<KP>, dim3(nblocks), dim3(kPtThreads), 0, s, blocks, ff, tf)
   switch (nodes) {
     case 2:
-      hipLaunchKernelGGL(k_transfer_linear, dim3(nblocks), dim3(kPtThreads), 0, s, blocks, ff, tf);
+      hipLaunchKernelGGL(k_transfer_points<2>, dim3(nblocks), dim3(kPtThreads), 0, s, blocks, ff, tf);
       break;
     case 3: OLL_TF(3); break;
     case 4: OLL_TF(4); break;

@@ -497,9 +497,10 @@ void launch_restrict_defect(hipStream_t s, const PtBlock *blocks, int nblocks, i
 // tf of their targets (multigrid::Transferir): PtBlock::mg packs the
 // region (bits 0-1), `all` (bit 2) and `to_zero` (bit 3); nodes = 2 for
 // linear interpolation, else the Lagrange nodes per axis (3..10); false
-// for other node counts
+// for other node counts.  tiles: a block is a tile of kXferTile points from
+// (i0, j0, k0) (Lagrange only), else nq points in lexicographic order
 bool launch_transfer_fields(hipStream_t s, const PtBlock *blocks, int nblocks, int ff, int tf,
-                            int nodes);
+                            int nodes, bool tiles);
 // v = full-weighting filter of the defect w (all points of the listed
 // boxes); runs = 1: blocks over runs of filter_run_length() points along x
 // (ceil(n0 / length) runs per row), 0: blocks over points
