@@ -875,6 +875,7 @@ struct Builder {
           L.order = order;
           L.eq = eq;
           L.colour = q;
+          L.first = s == 0 && q == 0 && nfused == 0 ? kFirstPass : 0;
           L.off = coff;
           L.n = int(cb.size());
           L.max_row = std::min(pc, threads);
@@ -1318,7 +1319,7 @@ int issue(const Schedule &S, hipStream_t s, Timing *t, std::string &err) {
         break;
       case Launch::SMOOTH:
         launch_smooth(s, reinterpret_cast<const RowBlock *>(items), L.n, L.max_row, L.order, L.eq,
-                      L.colour, L.threads, e0, e1, L.box1);
+                      L.colour + L.first, L.threads, e0, e1, L.box1);
         break;
       case Launch::DEFECT32:
         launch_defect32(s, reinterpret_cast<const RowBlock *>(items), L.n, L.max_row, L.order, L.eq);

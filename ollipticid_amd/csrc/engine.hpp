@@ -108,6 +108,7 @@ struct Launch {
   int threads = kRowThreads;  // colour passes: threads per workgroup
   int max_pts = 0, max_int = 0;  // COARSE: largest box, colour slot list; ROBIN: edge cross-sections
   int pair = 0, parity = 0;  // SMOOTH_FUSED: two passes or one; 0 reads u, 1 reads r
+  int first = 0;  // SMOOTH: kFirstPass for a phase's first pass, else 0
   double bytes = 0;   // algorithmic bytes (smoother launches, FP64 or FP32)
   const DevBox *box1 = nullptr;  // row launches over a single box: its descriptor
 };

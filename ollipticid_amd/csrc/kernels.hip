@@ -378,9 +378,12 @@ __device__ __forceinline__ double row_max_pos(double v) {
 // every block.  An atomic per block on 16 lines cost a colour pass of one
 // N=65 box 0.5 us of 4.4.  Only launches of small workgroups (sweep_rule)
 // read it: in longer launches the atomics overlap the passes, and the load
-// would cost 2%.
-__device__ __forceinline__ double norm_seen(const unsigned long long *slot) {
-  if (blockDim.x > kFewRowThreads || threadIdx.x != 0 || !slot) return 0.0;
+// would cost 2%.  Nor is it read in a phase's first pass, where every block
+// has its atomic and the load would wait for those before it (one sweep of a
+// 129^3 box, 2nd order: 78.5 us a call with the load, 70.2 without; 4th order
+// 86 and 74; unread in the whole first sweep 72 and 76).
+__device__ __forceinline__ double norm_seen(const unsigned long long *slot, bool first = false) {
+  if (first || blockDim.x > kFewRowThreads || threadIdx.x != 0 || !slot) return 0.0;
   return ld<double>(slot, (blockIdx.x & (kNormSubSlots - 1)) * (kNormStride * 8u));
 }
 
@@ -494,12 +497,13 @@ __device__ __forceinline__ Nbr<NC> box_offs(ConstBox &B, int c, int s) {
 // ------------------------------------------------------------------
 template <int ORD, int EQ>
 __device__ __forceinline__ void smooth_rows(const RowBlock &Bk, ConstBox &B, unsigned per_row,
-                                            float inv_per_row, int colour) {
+                                            float inv_per_row, int pass) {
+  const int colour = pass & (kFirstPass - 1);
   constexpr int R = ORD / 2;
   constexpr int NC = colours_of(ORD, EQ);
   const unsigned lr = fast_div(threadIdx.x, per_row, inv_per_row);
   const int t = int(threadIdx.x - lr * per_row);
-  const double seen = norm_seen(Bk.norm);
+  const double seen = norm_seen(Bk.norm, pass >= kFirstPass);
   double rmax = 0.0;
   unsigned p;
   int s, i, j, k;
@@ -653,12 +657,13 @@ __device__ __forceinline__ void point_op_pair(const SweepBox &B, unsigned o,
 
 template <int ORD, int EQ>
 __device__ __forceinline__ void smooth_pairs(const RowBlock &Bk, const SweepBox &B, unsigned per_row,
-                                             float inv_per_row, int colour) {
+                                             float inv_per_row, int pass) {
+  const int colour = pass & (kFirstPass - 1);
   constexpr int R = ORD / 2, NC = R + 1;
   const unsigned lr = fast_div(threadIdx.x, per_row, inv_per_row);
   unsigned t = threadIdx.x - lr * per_row;
   const int col = B.flip ? NC - 1 - colour : colour;
-  const double seen = norm_seen(Bk.norm);
+  const double seen = norm_seen(Bk.norm, pass >= kFirstPass);
   double rmax = 0.0;
   unsigned row = unsigned(Bk.row0) + lr;
   if (lr < unsigned(Bk.rows)) {
@@ -721,7 +726,7 @@ __global__ __launch_bounds__(kMaxRowThreads)
 __attribute__((amdgpu_waves_per_eu(sweep_points(EQ) == 2 ? 4 : 1, sweep_points(EQ) == 2 ? 4 : 8)))
 void k_smooth(const RowBlock *__restrict__ blocks,
                                                         unsigned per_row, float inv_per_row,
-                                                        int colour, const DevBox *box1) {
+                                                        int pass, const DevBox *box1) {
   if constexpr (sweep_points(EQ) == 2) {
     RowBlock Bk;
     SweepBox B;
@@ -734,12 +739,12 @@ void k_smooth(const RowBlock *__restrict__ blocks,
       B.load(cbox(Bk.box));
       B.wait();
     }
-    smooth_pairs<ORD, EQ>(Bk, B, per_row, inv_per_row, colour);
+    smooth_pairs<ORD, EQ>(Bk, B, per_row, inv_per_row, pass);
   } else {
     const RowBlock Bk = blocks[xcd_block()];
     const DevBox *box = box1 ? box1 : Bk.box;
     fetch_box(box);
-    smooth_rows<ORD, EQ>(Bk, cbox(box), per_row, inv_per_row, colour);
+    smooth_rows<ORD, EQ>(Bk, cbox(box), per_row, inv_per_row, pass);
   }
 }
 
@@ -3366,15 +3371,15 @@ __global__ void k_zero_lists(const ZeroItem *items) {
 inline unsigned ceil_div(long long a, long long b) { return unsigned((a + b - 1) / b); }
 
 template <int ORD, int EQ>
-void smooth_impl(hipStream_t s, const RowBlock *blocks, int nb, int per_row, int colour,
+void smooth_impl(hipStream_t s, const RowBlock *blocks, int nb, int per_row, int pass,
                  int threads, hipEvent_t e0, hipEvent_t e1, const DevBox *box1) {
   if (nb == 0) return;
   if (e0)  // timed (never under graph capture): the runtime stamps e0, e1
     hipExtLaunchKernelGGL((k_smooth<ORD, EQ>), dim3(nb), dim3(threads), 0, s, e0, e1, 0, blocks,
-                          unsigned(per_row), 1.0f / float(per_row), colour, box1);
+                          unsigned(per_row), 1.0f / float(per_row), pass, box1);
   else
     hipLaunchKernelGGL((k_smooth<ORD, EQ>), dim3(nb), dim3(threads), 0, s, blocks,
-                       unsigned(per_row), 1.0f / float(per_row), colour, box1);
+                       unsigned(per_row), 1.0f / float(per_row), pass, box1);
 }
 
 template <int ORD, int EQ>
@@ -3467,9 +3472,9 @@ bool set_sweep_threads(int mixed, int order, int threads) {
 }
 
 void launch_smooth(hipStream_t s, const RowBlock *blocks, int nblocks, int per_row, int order,
-                   int eq, int colour, int threads, hipEvent_t e0, hipEvent_t e1,
+                   int eq, int pass, int threads, hipEvent_t e0, hipEvent_t e1,
                    const DevBox *box1) {
-  OLL_DISPATCH_ORDER(order, eq, smooth_impl, s, blocks, nblocks, per_row, colour, threads, e0, e1,
+  OLL_DISPATCH_ORDER(order, eq, smooth_impl, s, blocks, nblocks, per_row, pass, threads, e0, e1,
                      box1);
 }
 
